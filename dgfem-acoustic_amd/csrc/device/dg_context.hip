@@ -79,6 +79,8 @@ struct dg_context;
 using StageFn = void (*)(dg_context*, int stage, const void* qin, void* qout, void* uout, bool snap);
 using PerStepFn = void (*)(dg_context*);
 using ClosureFn = void (*)(dg_context*, const void* qin);
+using PackFn = void (*)(dg_context*, const double* in, void* hi, void* lo);
+using UnpackFn = void (*)(dg_context*, const void* hi, const void* lo, double* out);
 using TraceFn = void (*)(dg_context*, int64_t n, const int64_t* elem, const int32_t* face, double* out,
                          double* normals);
 
@@ -96,7 +98,7 @@ struct dg_context {
     void *u = nullptr, *ulo = nullptr, *qa = nullptr, *qb = nullptr, *acc = nullptr, *snap = nullptr,
          *geo = nullptr, *fgeo = nullptr, *ops = nullptr;
     int32_t *nbr = nullptr, *iops = nullptr;
-    uint8_t* code = nullptr;
+    uint8_t *code = nullptr, *toCanon = nullptr;
     double* resPartial = nullptr;
     double* resGroup = nullptr;  // per-group residual sums when nblocks > 4 kResGroup
     int64_t nblocks = 0, nResGroups = 0;
@@ -154,6 +156,8 @@ struct dg_context {
     int64_t closureParams = 0;
     ClosureFn closureFn = nullptr;
     TraceFn traceFn = nullptr;
+    PackFn packFn = nullptr;
+    UnpackFn unpackFn = nullptr;
     // per-run settings read by the launchers
     int curResid = 1;
     double curDt = 0.0, gDt = -1.0;
@@ -530,8 +534,24 @@ void launchTraces(dg_context* c, int64_t n, const int64_t* elem, const int32_t* 
                        static_cast<const T*>(c->ops), c->iops, c->nbr, c->code, elem, face, n, out, normals);
 }
 
+template <int DIM, int P, int NF, typename T>
+void launchPack(dg_context* c, const double* in, void* hi, void* lo) {
+    const int64_t n = c->K * c->Np;
+    hipLaunchKernelGGL((dgk::packStateKernel<DIM, P, NF, T>), dim3(static_cast<unsigned>((n + 255) / 256)), dim3(256), 0,
+                       c->stream, in, c->toCanon, n, static_cast<T*>(hi), static_cast<T*>(lo));
+}
+
+template <int DIM, int P, int NF, typename T>
+void launchUnpack(dg_context* c, const void* hi, const void* lo, double* out) {
+    const int64_t n = c->K * c->Np;
+    hipLaunchKernelGGL((dgk::unpackStateKernel<DIM, P, NF, T>), dim3(static_cast<unsigned>((n + 255) / 256)), dim3(256),
+                       0, c->stream, static_cast<const T*>(hi), static_cast<const T*>(lo), c->toCanon, n, out);
+}
+
 template <int DIM, int P, int NF>
 void pickAux(dg_context* c) {
+    c->packFn = c->precision == DG_FP64 ? &launchPack<DIM, P, NF, double> : &launchPack<DIM, P, NF, float>;
+    c->unpackFn = c->precision == DG_FP64 ? &launchUnpack<DIM, P, NF, double> : &launchUnpack<DIM, P, NF, float>;
     if (c->precision == DG_FP64) {
         c->traceFn = &launchTraces<DIM, P, NF, double>;
         if constexpr (DIM == 2 || P <= 3) c->closureFn = &launchClosure<DIM, P, NF, double>;
@@ -931,24 +951,22 @@ void captureGraphs(dg_context* c, int integrator, bool resid, int steps) {
     c->gResid = resid ? 1 : 0;
 }
 
-// Caller layout [nf][K*Np] (file node order) <-> device layout [K][Np canonical][nf].
-void toDeviceLayout(const dg_context* c, const double* u, std::vector<double>& out) {
-    const int64_t N = c->K * c->Np;
-    out.assign(static_cast<size_t>(N) * c->nf, 0.0);
-    for (int64_t e = 0; e < c->K; ++e)
-        for (int a = 0; a < c->Np; ++a) {
-            const int64_t cn = e * c->Np + c->mesh.toCanon[e * c->Np + a];
-            for (int f = 0; f < c->nf; ++f) out[cn * c->nf + f] = u[f * N + e * c->Np + a];
-        }
+// Caller layout [nf][K*Np] (file node order) <-> device layout [K][Np canonical][nf] through the
+// device staging area `stage` (8 bytes per value): stage registers that hold nothing between steps.
+void writeState(dg_context* c, const double* u, void* stage, void* hi, void* lo) {
+    const size_t bytes = static_cast<size_t>(c->K) * c->Np * c->nf * sizeof(double);
+    HIPCHK(hipMemcpyAsync(stage, u, bytes, hipMemcpyHostToDevice, c->stream));
+    c->packFn(c, static_cast<const double*>(stage), hi, lo);
+    HIPCHK(hipGetLastError());
+    HIPCHK(hipStreamSynchronize(c->stream));
 }
 
-void fromDeviceLayout(const dg_context* c, const std::vector<double>& dev, double* u) {
-    const int64_t N = c->K * c->Np;
-    for (int64_t e = 0; e < c->K; ++e)
-        for (int a = 0; a < c->Np; ++a) {
-            const int64_t cn = e * c->Np + c->mesh.toCanon[e * c->Np + a];
-            for (int f = 0; f < c->nf; ++f) u[f * N + e * c->Np + a] = dev[cn * c->nf + f];
-        }
+void readState(dg_context* c, const void* hi, const void* lo, void* stage, double* u) {
+    const size_t bytes = static_cast<size_t>(c->K) * c->Np * c->nf * sizeof(double);
+    c->unpackFn(c, hi, lo, static_cast<double*>(stage));
+    HIPCHK(hipGetLastError());
+    HIPCHK(hipMemcpyAsync(u, stage, bytes, hipMemcpyDeviceToHost, c->stream));
+    HIPCHK(hipStreamSynchronize(c->stream));
 }
 
 void uploadState(dg_context* c, const std::vector<double>& dev, void* hiBuf, void* loBuf) {
@@ -988,7 +1006,7 @@ void destroyContext(dg_context* c) {
     if (c->device >= 0) (void)hipSetDevice(c->device);
     releaseGraphs(c);
     freeTables(c);
-    for (void* p : {c->u, c->ulo, c->qa, c->qb, c->acc, c->snap, c->geo, c->fgeo, c->ops, c->afrag, c->afragBf})
+    for (void* p : {c->u, c->ulo, c->qa, c->snap, c->geo, c->fgeo, c->ops, c->afrag, c->afragBf})  // qa: with acc, qb
         devFree(p);
     devFree(c->nbr);
     devFree(c->iops);
@@ -1107,9 +1125,12 @@ dg_status dg_create(const dg_mesh_desc* m, const dg_physics* ph, const dg_option
                                            : static_cast<void*>(devAlloc<float>(c, n));
         };
         c->u = alloc(nstate);
-        c->qa = alloc(nstate);
-        c->qb = alloc(nstate);
-        c->acc = alloc(nstate);
+        // the stage registers qa, acc, qb in one allocation: any two neighbours hold a state in the
+        // caller's FP64 (the staging area of writeState and readState)
+        const size_t reg = align256(nstate * c->tsize);
+        c->qa = devAlloc<unsigned char>(c, 3 * reg);
+        c->acc = static_cast<unsigned char*>(c->qa) + reg;
+        c->qb = static_cast<unsigned char*>(c->qa) + 2 * reg;
         // the residual snapshot holds the state's leading word only (mixed precision: the FP32
         // value nearest the compensated state, so a residual term is off by <= 2^-24 |snapshot|)
         c->snap = alloc(nstate);
@@ -1154,7 +1175,13 @@ dg_status dg_create(const dg_mesh_desc* m, const dg_physics* ph, const dg_option
         }
         c->iops = uploadVec(c, iops);
         c->nbr = uploadVec(c, c->mesh.nbr);
-        c->code = uploadVec(c, c->mesh.nbrCode);
+        // neighbour codes and, behind them, the caller's node positions (one allocation and copy)
+        std::vector<uint8_t> bytes(c->mesh.nbrCode);
+        bytes.resize(align256(bytes.size()));
+        const size_t codeBytes = bytes.size();
+        bytes.insert(bytes.end(), c->mesh.toCanon.begin(), c->mesh.toCanon.end());
+        c->code = uploadVec(c, bytes);
+        c->toCanon = c->code + codeBytes;
         c->nLearned = static_cast<int64_t>(c->mesh.learnedFaces.size());
         if (c->nLearned > 0) {
             c->dLearned = uploadVec(c, c->mesh.learnedFaces);
@@ -1289,9 +1316,7 @@ dg_status dg_set_state(dg_context* c, const double* u) {
     if (!c || !u) return DG_ERR_INVALID;
     try {
         HIPCHK(hipSetDevice(c->device));
-        std::vector<double> dev;
-        toDeviceLayout(c, u, dev);
-        uploadState(c, dev, c->u, c->ulo);
+        writeState(c, u, c->qa, c->u, c->ulo);
     } catch (const std::exception& ex) {
         return fail(c, DG_ERR_DEVICE, ex.what());
     }
@@ -1302,10 +1327,7 @@ dg_status dg_get_state(dg_context* c, double* u) {
     if (!c || !u) return DG_ERR_INVALID;
     try {
         HIPCHK(hipSetDevice(c->device));
-        HIPCHK(hipStreamSynchronize(c->stream));
-        std::vector<double> dev;
-        downloadState(c, c->u, c->ulo, dev);
-        fromDeviceLayout(c, dev, u);
+        readState(c, c->u, c->ulo, c->qa, u);
     } catch (const std::exception& ex) {
         return fail(c, DG_ERR_DEVICE, ex.what());
     }
@@ -1433,11 +1455,8 @@ dg_status dg_run(dg_context* c, const dg_run_params* prm, dg_step_fn on_step, dg
             if (isSave[done]) {
                 HIPCHK(hipMemcpyAsync(c->snap, c->u, stateN * c->tsize, hipMemcpyDeviceToDevice, c->stream));
                 if (on_save) {
-                    HIPCHK(hipStreamSynchronize(c->stream));
-                    std::vector<double> dev;
-                    downloadState(c, c->u, c->ulo, dev);
                     stateHost.resize(stateN);
-                    fromDeviceLayout(c, dev, stateHost.data());
+                    readState(c, c->u, c->ulo, c->qa, stateHost.data());
                     if (on_save(user, done, times[done], stateHost.data()) != 0) {
                         HIPCHK(hipEventDestroy(ev0));
                         HIPCHK(hipEventDestroy(ev1));
@@ -1546,16 +1565,11 @@ dg_status dg_rhs(dg_context* c, const double* u, double* k, double dt) {
     if (!c || !u || !k) return DG_ERR_INVALID;
     try {
         HIPCHK(hipSetDevice(c->device));
-        std::vector<double> dev;
-        toDeviceLayout(c, u, dev);
-        uploadState(c, dev, c->qa, nullptr);
+        writeState(c, u, c->acc, c->qa, nullptr);
         c->curDt = dt;
         runStage(c, dgk::kStageRHS, c->qa, c->qb, c->u, false);
         HIPCHK(hipGetLastError());
-        HIPCHK(hipStreamSynchronize(c->stream));
-        std::vector<double> out;
-        downloadState(c, c->qb, nullptr, out);
-        fromDeviceLayout(c, out, k);
+        readState(c, c->qb, nullptr, c->qa, k);
     } catch (const std::exception& ex) {
         return fail(c, DG_ERR_DEVICE, ex.what());
     }
