@@ -22,6 +22,7 @@
 #include "dg_closure.hpp"
 #include "dg_kernels.hpp"
 #include "dg_kernels_bf16.hpp"
+#include "dg_resident.hpp"
 
 namespace {
 
@@ -126,6 +127,15 @@ struct dg_context {
     double *hT = nullptr, *hV = nullptr, *hRes = nullptr, *hObs = nullptr;
     uint8_t* hVF = nullptr;
     bool tablesDirty = true;
+    // resident time loop (0 blocks: not used for this grid)
+    int64_t resBlocks = 0;
+    int resShape = 0;                  // dgk::kRes*
+    int resChunk = 0;                  // steps per launch
+    unsigned char* resMail = nullptr;  // two sets of mailboxes, then outcomes and counts per chunk
+    size_t resMailBytes = 0;           //   of one set
+    int *resOutcome = nullptr, *resDone = nullptr;
+    int32_t *dObsOff = nullptr, *dObsEntry = nullptr, *dObsSrc = nullptr;
+    double *resSteps = nullptr, *dObsVal = nullptr, *dSrcVal = nullptr;
     // graphs
     hipGraphExec_t gMulti = nullptr, gOne = nullptr;
     int gSteps = 0, gIntegrator = -1, gResid = -1;
@@ -754,8 +764,11 @@ void releaseGraphs(dg_context* c) {
 void freeTables(dg_context* c) {
     for (void* p : {static_cast<void*>(c->dSrcNodes), static_cast<void*>(c->dSrcLast), static_cast<void*>(c->dSrcCoverOff),
                     static_cast<void*>(c->dSrcCover), static_cast<void*>(c->dSrcParams), static_cast<void*>(c->dObsIdx),
-                    static_cast<void*>(c->dObsW), static_cast<void*>(c->dObsSeg0), static_cast<void*>(c->dSegPartial)})
+                    static_cast<void*>(c->dObsW), static_cast<void*>(c->dObsSeg0), static_cast<void*>(c->dSegPartial),
+                    static_cast<void*>(c->dObsOff), static_cast<void*>(c->dObsVal)})
         devFree(p);
+    c->dObsOff = c->dObsEntry = c->dObsSrc = nullptr;
+    c->dObsVal = nullptr;
     c->dSrcNodes = c->dSrcCoverOff = c->dObsIdx = nullptr;
     c->dSrcLast = c->dSrcCover = c->dObsSeg0 = nullptr;
     c->dSrcParams = c->dObsW = c->dSegPartial = nullptr;
@@ -767,6 +780,45 @@ V* uploadVec(dg_context* c, const std::vector<V>& v) {
     V* d = devAlloc<V>(c, v.size());
     if (!v.empty()) HIPCHK(hipMemcpy(d, v.data(), v.size() * sizeof(V), hipMemcpyHostToDevice));
     return d;
+}
+
+// Observer tables of the resident time loop: per block the entries (thread, slot) of its nodes,
+// threads ascending, and per slot (256 per segment) the slot that holds its value. obsVal takes at
+// most kResObsBytes: with many observer nodes a launch does fewer steps.
+constexpr size_t kResObsBytes = size_t(16) << 20;
+constexpr int kResMaxChunk = 256, kResMinChunk = 16;
+
+void syncResidentTables(dg_context* c) {
+    const int64_t nodes = static_cast<int64_t>(dgk::residentElements(c->dim, c->p, c->resShape)) * c->Np;  // per block
+    const size_t slots = static_cast<size_t>(c->nseg) * 256;
+    std::vector<std::array<int32_t, 3>> ent;  // block, thread, slot
+    std::vector<int32_t> src;
+    for (const std::vector<int64_t>& nd : c->obsNodes)
+        for (size_t b = 0; b < nd.size(); b += 256) {
+            const int32_t first = static_cast<int32_t>(src.size());
+            for (size_t q = 0; q < 256; ++q) {
+                const bool in = b + q < nd.size();
+                const int32_t slot = static_cast<int32_t>(src.size());
+                if (in) ent.push_back({static_cast<int32_t>(nd[b + q] / nodes), static_cast<int32_t>(nd[b + q] % nodes), slot});
+                src.push_back(in ? slot : first);
+            }
+        }
+    std::sort(ent.begin(), ent.end());
+    // one array: offsets [blocks + 1], entries, sources
+    std::vector<int32_t> all(c->resBlocks + 1, 0);
+    for (const auto& e : ent) ++all[e[0] + 1];
+    for (int64_t b = 0; b < c->resBlocks; ++b) all[b + 1] += all[b];
+    const size_t nEnt = ent.size();
+    for (const auto& e : ent) all.insert(all.end(), {e[1], e[2]});
+    all.insert(all.end(), src.begin(), src.end());
+    c->dObsOff = uploadVec(c, all);
+    c->dObsEntry = c->dObsOff + c->resBlocks + 1;
+    c->dObsSrc = c->dObsEntry + 2 * nEnt;
+    c->resChunk = kResMaxChunk;
+    if (slots > 0) {
+        c->resChunk = static_cast<int>(std::min<size_t>(kResMaxChunk, kResObsBytes / (slots * 32)));
+        if (c->resChunk >= kResMinChunk) c->dObsVal = devAlloc<double>(c, c->resChunk * slots * 4);
+    }
 }
 
 void syncTables(dg_context* c) {
@@ -833,6 +885,7 @@ void syncTables(dg_context* c) {
     c->dObsW = uploadVec(c, ow);
     c->dObsSeg0 = uploadVec(c, obsSeg0);
     c->dSegPartial = devAlloc<double>(c, std::max(1, c->nseg) * 5);
+    if (c->resBlocks > 0) syncResidentTables(c);
     // rings and per-step tables
     const int64_t ns = std::max<int64_t>(1, static_cast<int64_t>(c->srcNodes.size()));
     const int64_t no = std::max<int64_t>(1, static_cast<int64_t>(c->obsNodes.size()));
@@ -840,9 +893,12 @@ void syncTables(dg_context* c) {
     devFree(c->dV);
     devFree(c->dVF);
     devFree(c->obsRing);
+    devFree(c->dSrcVal);
+    c->dSrcVal = nullptr;
     if (c->hV) (void)hipHostFree(c->hV);
     if (c->hVF) (void)hipHostFree(c->hVF);
     if (c->hObs) (void)hipHostFree(c->hObs);
+    if (c->resBlocks > 0 && !c->srcNodes.empty()) c->dSrcVal = devAlloc<double>(c, c->ringSlots * ns * 2);
     c->dT = devAlloc<double>(c, c->ringSlots);
     c->dV = devAlloc<double>(c, c->ringSlots * ns);
     c->dVF = devAlloc<uint8_t>(c, c->ringSlots * ns);
@@ -951,6 +1007,120 @@ void captureGraphs(dg_context* c, int integrator, bool resid, int steps) {
     c->gResid = resid ? 1 : 0;
 }
 
+// Grids that run in the resident time loop (dg_resident.hpp): at most as many 256-thread blocks as
+// the chip holds at once, on meshes without learned faces (their exterior states come from a kernel
+// of their own before every stage) and without an explicit DGFEM_KERNEL or DGFEM_POST_BRANCH (both
+// ask for launches per stage). DGFEM_RESIDENT=0 switches it off.
+void pickResident(dg_context* c) {
+    const char* env = std::getenv("DGFEM_RESIDENT");
+    if (c->nLearned > 0 || (env && env[0] == '0')) return;
+    for (const char* name : {"DGFEM_KERNEL", "DGFEM_POST_BRANCH"}) {
+        const char* v = std::getenv(name);
+        if (v && v[0]) return;
+    }
+    if (c->kernelKind != DG_KERNEL_VALU && c->kernelKind != DG_KERNEL_VM) return;
+    int cus = 0, coop = 0;
+    HIPCHK(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, c->device));
+    HIPCHK(hipDeviceGetAttribute(&coop, hipDeviceAttributeCooperativeLaunch, c->device));
+    if (!coop) return;
+    int64_t n = 0;
+    for (int shape = 0; shape < dgk::kResShapes; ++shape) {
+        const int eb = dgk::residentElements(c->dim, c->p, shape);
+        if (eb == 0) return;
+        n = (c->K + eb - 1) / eb;
+        c->resShape = shape;
+        if (n <= static_cast<int64_t>(cus) * dgk::residentBlocksPerCu(c->dim, c->p, c->nf, c->precision == DG_FP64, shape)) {
+            c->resBlocks = n;
+            break;
+        }
+    }
+    if (c->resBlocks == 0) return;
+    const size_t chunks = c->ringSlots / kResMinChunk, partials = static_cast<size_t>(kResMaxChunk) * n * 5;
+    c->resMailBytes = align256(static_cast<size_t>(c->K) * c->Nfc * c->Nfp * c->nf * c->tsize);
+    c->resMail = devAlloc<unsigned char>(c, 2 * c->resMailBytes + partials * 8 + 2 * chunks * sizeof(int));
+    c->resSteps = reinterpret_cast<double*>(c->resMail + 2 * c->resMailBytes);
+    c->resOutcome = reinterpret_cast<int*>(c->resSteps + partials);
+    c->resDone = c->resOutcome + chunks;
+}
+
+template <typename T>
+hipError_t launchChunk(dg_context* c, int chunk, int64_t slot0, int steps, int64_t batch, int integrator, bool resid) {
+    dgk::ResidentArgs<T> a{};
+    a.u = static_cast<T*>(c->u);
+    a.ulo = static_cast<T*>(c->ulo);
+    a.snap = resid ? static_cast<const T*>(c->snap) : nullptr;
+    a.mail = reinterpret_cast<T*>(c->resMail);
+    a.mailBytes = static_cast<int>(c->resMailBytes);
+    a.geo = static_cast<const T*>(c->geo);
+    a.fgeo = static_cast<const T*>(c->fgeo);
+    a.nbr = c->nbr;
+    a.code = c->code;
+    a.ops = static_cast<const T*>(c->ops);
+    a.iops = c->iops;
+    a.outcome = c->resOutcome;
+    a.done = c->resDone;
+    a.resPartial = c->resSteps;
+    a.obsOff = c->dObsOff;
+    a.obsEntry = c->dObsEntry;
+    a.obsVal = c->dObsVal;
+    a.srcVal = c->dSrcVal;
+    a.nonfinite = c->nonfinite;
+    a.K = c->K;
+    a.slot0 = slot0;
+    a.batchSteps = batch;
+    const char* env = std::getenv("DGFEM_RESIDENT_PATIENCE");  // microseconds; 0: no wait at all
+    a.patience = env && env[0] ? std::strtoull(env, nullptr, 10) * 100 : 200000000ull;  // 2 s
+    a.dt = static_cast<T>(c->curDt);
+    a.steps = steps;
+    a.chunk = chunk;
+    a.slots = c->nseg * 256;
+    a.euler = integrator == DG_EULER;
+    a.ph = makePhysics<T>(c->phys);
+    return dgk::launchResident<T>(c->dim, c->p, c->nf, c->resShape, a, sourceArgs(c), static_cast<unsigned>(c->resBlocks), c->stream);
+}
+
+// Enqueues a batch of n steps (state, step tables and counters set) in the resident time loop;
+// returns the number of chunks.
+int launchResidentBatch(dg_context* c, int64_t n, int integrator, bool resid) {
+    const int chunks = static_cast<int>((n + c->resChunk - 1) / c->resChunk);
+    const int64_t ns = static_cast<int64_t>(c->srcNodes.size());
+    if (ns > 0)
+        hipLaunchKernelGGL(dgk::residentSourceKernel, dim3(static_cast<unsigned>((n * ns + 255) / 256)), dim3(256), 0,
+                           c->stream, sourceArgs(c), n, c->dSrcVal);
+    for (int k = 0; k < chunks; ++k) {
+        const int64_t s0 = static_cast<int64_t>(k) * c->resChunk;
+        const int steps = static_cast<int>(std::min<int64_t>(c->resChunk, n - s0));
+        const int64_t words = static_cast<int64_t>(2 * c->resMailBytes / 16), clear = std::max<int64_t>(words, chunks);
+        hipLaunchKernelGGL(dgk::residentResetKernel, dim3(static_cast<unsigned>((clear + 255) / 256)), dim3(256), 0,
+                           c->stream, reinterpret_cast<uint4*>(c->resMail), words, c->resOutcome, c->resDone,
+                           k == 0 ? chunks : 0);
+        if ((c->precision == DG_FP64 ? launchChunk<double>(c, k, s0, steps, n, integrator, resid)
+                                     : launchChunk<float>(c, k, s0, steps, n, integrator, resid)) != hipSuccess) {
+            (void)hipGetLastError();  // not launched: its outcome stays kPending
+            break;
+        }
+        dgk::ResidentPostArgs p{};
+        p.resPartial = c->resSteps;
+        p.nblocks = c->resBlocks;
+        p.invN = 1.0 / static_cast<double>(c->K * c->Np);
+        p.obsVal = c->dObsVal;
+        p.obsW = c->dObsW;
+        p.obsSrc = c->dObsSrc;
+        p.obsSeg0 = c->dObsSeg0;
+        p.nseg = c->nseg;
+        p.nobs = static_cast<int>(c->obsNodes.size());
+        p.slots = c->nseg * 256;
+        p.resRing = c->resRing;
+        p.obsRing = c->obsRing;
+        p.nonfinite = c->nonfinite;
+        p.outcome = c->resOutcome + k;
+        p.slot0 = s0;
+        p.computeResiduals = resid ? 1 : 0;
+        hipLaunchKernelGGL(dgk::residentPostKernel, dim3(steps), dim3(dgk::kPostBlock), 0, c->stream, p);
+    }
+    return chunks;
+}
+
 // Caller layout [nf][K*Np] (file node order) <-> device layout [K][Np canonical][nf] through the
 // device staging area `stage` (8 bytes per value): stage registers that hold nothing between steps.
 void writeState(dg_context* c, const double* u, void* stage, void* hi, void* lo) {
@@ -1025,6 +1195,8 @@ void destroyContext(dg_context* c) {
     devFree(c->dLearned);
     devFree(c->ghost);
     devFree(c->dClosureW);
+    devFree(c->resMail);
+    devFree(c->dSrcVal);
     for (void* h : {static_cast<void*>(c->hT), static_cast<void*>(c->hV), static_cast<void*>(c->hRes),
                     static_cast<void*>(c->hObs), static_cast<void*>(c->hVF)})
         if (h) (void)hipHostFree(h);
@@ -1204,6 +1376,7 @@ dg_status dg_create(const dg_mesh_desc* m, const dg_physics* ph, const dg_option
         c->srcBase = devAlloc<int64_t>(c, 1);
         HIPCHK(hipHostMalloc(reinterpret_cast<void**>(&c->hT), sizeof(double) * c->ringSlots));
         HIPCHK(hipHostMalloc(reinterpret_cast<void**>(&c->hRes), sizeof(double) * c->ringSlots * 5));
+        pickResident(c);
         c->tablesDirty = true;
         syncTables(c);
         HIPCHK(hipDeviceSynchronize());
@@ -1435,9 +1608,23 @@ dg_status dg_run(dg_context* c, const dg_run_params* prm, dg_step_fn on_step, dg
         c->curResid = resid ? 1 : 0;
         c->curDt = prm->dt;
         const bool useGraph = c->opt.use_graph != 0;
-        if (useGraph && (c->gOne == nullptr || c->gIntegrator != prm->integrator || c->gResid != (resid ? 1 : 0) ||
-                         c->gSteps != c->opt.steps_per_graph || c->gDt != prm->dt))
-            captureGraphs(c, prm->integrator, resid, c->opt.steps_per_graph), c->gDt = prm->dt;
+        const bool resident = c->resBlocks > 0 && c->resChunk >= kResMinChunk;
+        auto readyGraphs = [&] {
+            if (useGraph && (c->gOne == nullptr || c->gIntegrator != prm->integrator || c->gResid != (resid ? 1 : 0) ||
+                             c->gSteps != c->opt.steps_per_graph || c->gDt != prm->dt))
+                captureGraphs(c, prm->integrator, resid, c->opt.steps_per_graph), c->gDt = prm->dt;
+        };
+        // steps s .. n-1 of a batch, launched kernel by kernel
+        auto launchSteps = [&](int64_t s, int64_t n) {
+            if (useGraph) {
+                if (c->gMulti)
+                    for (; s + c->gSteps <= n; s += c->gSteps) HIPCHK(hipGraphLaunch(c->gMulti, c->stream));
+                for (; s < n; ++s) HIPCHK(hipGraphLaunch(c->gOne, c->stream));
+            } else {
+                for (; s < n; ++s) launchStep(c, prm->integrator, resid);
+            }
+        };
+        if (!resident) readyGraphs();
         const int64_t nsteps = static_cast<int64_t>(times.size());
         const int ns = static_cast<int>(c->srcNodes.size());
         const int no = static_cast<int>(c->obsNodes.size());
@@ -1447,6 +1634,7 @@ dg_status dg_run(dg_context* c, const dg_run_params* prm, dg_step_fn on_step, dg
         HIPCHK(hipEventCreate(&ev1));
         double devMs = 0.0;
         std::vector<double> stateHost;
+        std::vector<int> outcome;
         int64_t done = 0;
         while (done < nsteps) {
             int64_t end = done + 1;
@@ -1480,16 +1668,25 @@ dg_status dg_run(dg_context* c, const dg_run_params* prm, dg_step_fn on_step, dg
                 HIPCHK(hipMemcpyAsync(c->dVF, c->hVF, n * ns, hipMemcpyHostToDevice, c->stream));
             }
             hipLaunchKernelGGL(dgk::setCounterKernel, dim3(1), dim3(1), 0, c->stream, c->counter, c->batchSteps,
-                               n, c->nonfinite, c->srcBase);
+                               n, c->nonfinite, c->srcBase, int64_t(0));
             HIPCHK(hipEventRecord(ev0, c->stream));
             c->sourceFn(c);
-            if (useGraph) {
-                int64_t s = 0;
-                if (c->gMulti)
-                    for (; s + c->gSteps <= n; s += c->gSteps) HIPCHK(hipGraphLaunch(c->gMulti, c->stream));
-                for (; s < n; ++s) HIPCHK(hipGraphLaunch(c->gOne, c->stream));
+            if (resident) {
+                outcome.assign(launchResidentBatch(c, n, prm->integrator, resid), dgk::kPending);
+                HIPCHK(hipMemcpyAsync(outcome.data(), c->resOutcome, outcome.size() * sizeof(int), hipMemcpyDeviceToHost,
+                                      c->stream));
+                HIPCHK(hipStreamSynchronize(c->stream));
+                const int64_t good = std::find_if(outcome.begin(), outcome.end(), [](int o) { return o != dgk::kDone; }) -
+                                     outcome.begin();
+                if (good < static_cast<int64_t>(outcome.size())) {
+                    // a block waited too long: the state is the one before chunk `good`
+                    readyGraphs();
+                    hipLaunchKernelGGL(dgk::setCounterKernel, dim3(1), dim3(1), 0, c->stream, c->counter, c->batchSteps, n,
+                                       c->nonfinite, c->srcBase, good * c->resChunk);
+                    launchSteps(good * c->resChunk, n);
+                }
             } else {
-                for (int64_t s = 0; s < n; ++s) launchStep(c, prm->integrator, resid);
+                launchSteps(0, n);
             }
             HIPCHK(hipGetLastError());
             HIPCHK(hipEventRecord(ev1, c->stream));
@@ -1610,7 +1807,7 @@ dg_status dg_profile_steps(dg_context* c, double dt, int32_t steps, double* stag
         for (size_t s = 0; s < tt.size(); ++s) c->hT[s] = s * dt;
         HIPCHK(hipMemcpyAsync(c->dT, c->hT, sizeof(double) * tt.size(), hipMemcpyHostToDevice, c->stream));
         hipLaunchKernelGGL(dgk::setCounterKernel, dim3(1), dim3(1), 0, c->stream, c->counter, c->batchSteps,
-                           static_cast<int64_t>(tt.size()), c->nonfinite, c->srcBase);
+                           static_cast<int64_t>(tt.size()), c->nonfinite, c->srcBase, int64_t(0));
         std::vector<hipEvent_t> ev(14);
         for (auto& e : ev) HIPCHK(hipEventCreate(&e));
         double acc[6] = {0, 0, 0, 0, 0, 0};

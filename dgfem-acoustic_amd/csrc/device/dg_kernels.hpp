@@ -1834,12 +1834,13 @@ __global__ __launch_bounds__(kPostBlock) void postKernel(PostArgs p, SourceArgs 
 }
 
 [[maybe_unused]] static __global__ void setCounterKernel(int64_t* counter, int64_t* batchSteps, int64_t nsteps, int* flag,
-                                                         int64_t* srcBase) {
-    *counter = 0;
+                                                         int64_t* srcBase, int64_t first) {
+    // `first` > 0: the batch goes on at that step (what earlier steps reported stays)
+    *counter = first;
     *batchSteps = nsteps;
-    flag[0] = -1;
+    if (first == 0) flag[0] = -1;
     flag[1] = 0;
-    *srcBase = 0;
+    *srcBase = first;
 }
 
 // Source overwrite of step `*base + offset` of the batch (when that step exists) inside a captured
