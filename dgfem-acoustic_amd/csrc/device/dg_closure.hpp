@@ -164,6 +164,202 @@ __device__ inline void mlpForwardWave(const float* net, const float* sx, float* 
     waveFence();
 }
 
+// ------------------------------------------- the network on the matrix cores, 16 faces ----
+//
+// Exterior states of 16 faces by a block of 4 waves. The three layers are products of BF16 weights
+// (exact operands) with FP32 activations split into three BF16 terms (FP32 operand precision) on
+// v_mfma_f32_16x16x32_bf16, FP32 accumulation from the bias on, the small terms summed apart and
+// added once (see mfmaSplit); a column is a face, wave w owns hidden units 16 w .. 16 w + 15. Bound by
+// the latency of the chain (three products of 3-6 instructions, two tanh, three exchanges through
+// LDS), so the weights are registers of their lanes. One wave evaluating 4 or 8 faces with a lane per
+// hidden unit and the weights in LDS took 7.2 us (400 faces, order 4 triangles) and 12.1 us
+// (6,912 faces, order 3 tetrahedra) per launch; this takes 4.7 and 6.5, and is as exact or more
+// (FP64 runs with a random network, 100 steps, against 64 bits: 1.5e-10 and 1.9e-10; 3.2e-10 and
+// 5.1e-10 with the wave-per-face kernel).
+
+constexpr int kTileFaces = 16;
+constexpr int kClosureBlock = 256;
+
+// Operand words of the network as one array (see packClosure): A fragments of layer 1 [4 row
+// tiles][64 lanes], layer 2 [4][2 k-steps][64], layer 3 [2][64], 8 BF16 each, then the biases of
+// layers 1, 2, 3 in FP32 (64, 64, 16).
+constexpr int kFrag1 = 4 * 64, kFrag2 = 4 * 2 * 64, kFrag3 = 2 * 64;
+constexpr int kNetWords = kFrag1 + kFrag2 + kFrag3 + (64 + 64 + 16) / 4;  // of 16 bytes
+
+inline void packClosure(int nin, int nout, const uint16_t* w, uint32_t* out) {
+    const uint16_t *w1 = w, *b1 = w1 + kH * nin, *w2 = b1 + kH, *b2 = w2 + kH * kH, *w3 = b2 + kH, *b3 = w3 + nout * kH;
+    uint16_t* h = reinterpret_cast<uint16_t*>(out);
+    auto put = [&](const uint16_t* m, int rows, int cols, int row0, int col0) {
+        for (int lane = 0; lane < 64; ++lane)
+            for (int j = 0; j < 8; ++j, ++h) {
+                const int r = row0 + lane % 16, c = col0 + 8 * (lane / 16) + j;
+                *h = r < rows && c < cols ? m[r * cols + c] : uint16_t(0);
+            }
+    };
+    for (int t = 0; t < 4; ++t) put(w1, kH, nin, 16 * t, 0);
+    for (int t = 0; t < 4; ++t)
+        for (int ks = 0; ks < 2; ++ks) put(w2, kH, kH, 16 * t, 32 * ks);
+    for (int ks = 0; ks < 2; ++ks) put(w3, nout, kH, 0, 32 * ks);
+    float* f = reinterpret_cast<float*>(h);
+    for (int i = 0; i < kH; ++i) *f++ = bf16ToFloat(b1[i]);
+    for (int i = 0; i < kH; ++i) *f++ = bf16ToFloat(b2[i]);
+    for (int i = 0; i < 16; ++i) *f++ = i < nout ? bf16ToFloat(b3[i]) : 0.0f;
+}
+
+struct ClosureNet {
+    dgk::u32x4_t a1, a2[2], a3[2];
+    dgk::f32x4_t b1, b2, b3;
+};
+
+__device__ inline ClosureNet loadClosureNet(const dgk::u32x4_t* __restrict__ w, int wave, int lane) {
+    const dgk::f32x4_t* b = reinterpret_cast<const dgk::f32x4_t*>(w + kFrag1 + kFrag2 + kFrag3);
+    const int g = lane >> 4;
+    ClosureNet n;
+    n.a1 = w[wave * 64 + lane];
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks) {
+        n.a2[ks] = w[kFrag1 + (wave * 2 + ks) * 64 + lane];
+        n.a3[ks] = w[kFrag1 + kFrag2 + ks * 64 + lane];
+    }
+    n.b1 = b[4 * wave + g];  // rows 16 wave + 4 g + r of this lane's results
+    n.b2 = b[16 + 4 * wave + g];
+    n.b3 = b[32 + g];
+    return n;
+}
+
+struct ClosureLds {
+    static constexpr int kStride = kH + 4;
+    float x[kTileFaces * kStride];  // inputs, then second activations
+    float a[kTileFaces * kStride];  // first activations
+    float y[kTileFaces * 20];
+};
+
+// c += A . v for 8 FP32 values of the lane's column: the three BF16 terms of v, the small ones
+// summed apart (corr).
+__device__ inline void netProduct(dgk::u32x4_t A, const float* __restrict__ p, dgk::f32x4_t& c, dgk::f32x4_t& corr) {
+    const dgk::f32x4_t lo = *reinterpret_cast<const dgk::f32x4_t*>(p), hi = *reinterpret_cast<const dgk::f32x4_t*>(p + 4);
+    const float v[8] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
+    dgk::u32x4_t t[3];
+    dgk::splitFrag<3>(v, t);
+    corr = dgk::mfmaBf16(A, t[2], corr);
+    corr = dgk::mfmaBf16(A, t[1], corr);
+    c = dgk::mfmaBf16(A, t[0], c);
+}
+
+// Exterior state qp of face node (face slot tid / 16, node tid % 16; nodes past NFP idle) from its
+// interior state qm and the face's unit normal n. Called by all 256 threads of a block; begins
+// writing s.x and ends reading s.y, so calls in a row need no barrier between them.
+template <int DIM, int NFP, int NF, typename T>
+__device__ inline void closureExterior(const ClosureNet& w, ClosureLds& s, const dgk::Physics<T>& ph, const T (&n)[3],
+                                       const T (&qm)[NF], T (&qp)[NF]) {
+    constexpr int NT = DIM - 1;  // tangential directions
+    constexpr int NIN = DIM * NFP + 2, KS = ClosureLds::kStride;
+    static_assert(NFP < 15 && NIN <= 32, "16 lanes per face, one k-step of inputs");
+    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+    const int slot = tid >> 4, node = tid & 15;
+    const bool nodeLane = node < NFP;
+    const T c0 = ph.c0;
+    T t[NT][3], vn0, vt0;
+    if constexpr (DIM == 2) {
+        t[0][0] = -n[1];
+        t[0][1] = n[0];
+        t[0][2] = T(0);
+        vn0 = ph.v0[0] * n[0] + ph.v0[1] * n[1];
+        vt0 = ph.v0[0] * t[0][0] + ph.v0[1] * t[0][1];
+    } else {
+        vn0 = ph.v0[0] * n[0] + ph.v0[1] * n[1] + ph.v0[2] * n[2];
+        // t1 along the tangential mean flow, else along the axis least aligned with n
+        T u[3];
+        for (int c = 0; c < 3; ++c) u[c] = ph.v0[c] - vn0 * n[c];
+        vt0 = sqrt(u[0] * u[0] + u[1] * u[1] + u[2] * u[2]);
+        if (!(vt0 > T(1e-6) * c0)) {
+            const T ax = fabs(n[0]), ay = fabs(n[1]), az = fabs(n[2]);
+            const int k = (ax <= ay && ax <= az) ? 0 : (ay <= az ? 1 : 2);
+            const T nk = k == 0 ? n[0] : k == 1 ? n[1] : n[2];
+            for (int c = 0; c < 3; ++c) u[c] = (c == k ? T(1) : T(0)) - nk * n[c];
+            vt0 = T(0);
+        }
+        const T iu = T(1) / sqrt(u[0] * u[0] + u[1] * u[1] + u[2] * u[2]);
+        for (int c = 0; c < 3; ++c) t[0][c] = u[c] * iu;
+        t[NT - 1][0] = n[1] * t[0][2] - n[2] * t[0][1];
+        t[NT - 1][1] = n[2] * t[0][0] - n[0] * t[0][2];
+        t[NT - 1][2] = n[0] * t[0][1] - n[1] * t[0][0];
+    }
+    const T Pv = qm[0] * ph.irc0;
+    T Nn = qm[1] * n[0] + qm[2] * n[1];
+    if constexpr (DIM == 3) Nn += qm[3] * n[2];
+    const T wo = nodeLane ? Pv + Nn : T(0), wi = Pv - Nn;
+    T tt[NT];
+    for (int c = 0; c < NT; ++c) {
+        T v = qm[1] * t[c][0] + qm[2] * t[c][1];
+        if constexpr (DIM == 3) v += qm[3] * t[c][2];
+        tt[c] = nodeLane ? v : T(0);
+    }
+    // scale: RMS over the face's nodes of the outgoing and tangential characteristics
+    const float wof = static_cast<float>(wo);
+    float ss = wof * wof;
+    for (int c = 0; c < NT; ++c) {
+        const float ttf = static_cast<float>(tt[c]);
+        ss += ttf * ttf;
+    }
+#pragma unroll
+    for (int off = 8; off > 0; off >>= 1) ss += __shfl_xor(ss, off, 64);
+    const float sc = sqrtf(ss / NFP) + 1e-30f;
+    const float is = 1.0f / sc;
+    float* x = s.x + slot * KS;
+    if (nodeLane) {
+        x[node] = wof * is;
+        for (int c = 0; c < NT; ++c) x[(1 + c) * NFP + node] = static_cast<float>(tt[c]) * is;
+    } else if (node == NFP) {
+        const float ic0 = static_cast<float>(T(1) / c0);
+        x[DIM * NFP] = static_cast<float>(vn0) * ic0;
+        x[DIM * NFP + 1] = static_cast<float>(vt0) * ic0;
+    } else {
+        for (int i = NIN + node - NFP - 1; i < 32; i += 15 - NFP) x[i] = 0.0f;
+    }
+    __syncthreads();
+    const int col = lane & 15, g = lane >> 4, row = 16 * wave + 4 * g;
+    const dgk::f32x4_t zero = {0.0f, 0.0f, 0.0f, 0.0f};
+    {
+        dgk::f32x4_t z = w.b1, corr = zero;
+        netProduct(w.a1, &s.x[col * KS + 8 * g], z, corr);
+        z = z + corr;
+        *reinterpret_cast<dgk::f32x4_t*>(&s.a[col * KS + row]) = dgk::f32x4_t{tanhf(z.x), tanhf(z.y), tanhf(z.z), tanhf(z.w)};
+    }
+    __syncthreads();
+    {
+        dgk::f32x4_t z = w.b2, corr = zero;
+#pragma unroll
+        for (int ks = 0; ks < 2; ++ks) netProduct(w.a2[ks], &s.a[col * KS + 32 * ks + 8 * g], z, corr);
+        z = z + corr;
+        *reinterpret_cast<dgk::f32x4_t*>(&s.x[col * KS + row]) = dgk::f32x4_t{tanhf(z.x), tanhf(z.y), tanhf(z.z), tanhf(z.w)};
+    }
+    __syncthreads();
+    {
+        // every wave the outputs of all faces; it keeps those of its own four
+        dgk::f32x4_t z = w.b3, corr = zero;
+#pragma unroll
+        for (int ks = 0; ks < 2; ++ks) netProduct(w.a3[ks], &s.x[col * KS + 32 * ks + 8 * g], z, corr);
+        z = z + corr;
+        if ((col >> 2) == wave) *reinterpret_cast<dgk::f32x4_t*>(&s.y[col * 20 + 4 * g]) = z;
+    }
+    __syncthreads();
+    const T what = static_cast<T>(sc * s.y[slot * 20 + node]);
+    const T lam = vn0 - c0;
+    const T wip = (T(2) * lam * what - (lam + c0) * wi) / (lam - c0);
+    T tp[NT];
+    for (int c = 0; c < NT; ++c) tp[c] = (vn0 >= T(0)) ? tt[c] : -(vn0 + c0) * tt[c] / (vn0 - c0);
+    const T Pp = T(0.5) * (wo + wip), Np_ = T(0.5) * (wo - wip);
+    qp[0] = ph.rho0 * c0 * Pp;
+    for (int c = 0; c < DIM; ++c) {
+        T v = Np_ * n[c];
+        for (int k = 0; k < NT; ++k) v += tp[k] * t[k][c];
+        qp[1 + c] = v;
+    }
+    if constexpr (DIM == 2) qp[3] = qm[3];
+    if constexpr (NF == 5) qp[4] = qm[4] + (qp[0] - qm[0]) * ph.ic2;
+}
+
 template <typename T>
 struct ClosureArgs {
     const T* __restrict__ qin;          // stage input [K][NP][NF]
@@ -171,232 +367,30 @@ struct ClosureArgs {
     const T* __restrict__ fgeo;         // [K][NFC][4] outward unit normal, Fscale
     const int32_t* __restrict__ iops;   // fmask
     const int64_t* __restrict__ faces;  // element * NFC + local face
-    const uint16_t* __restrict__ w;     // BF16 parameters
+    const dgk::u32x4_t* __restrict__ w; // network (packClosure)
     int64_t nfaces;
     dgk::Physics<T> ph;
 };
 
-// Forward pass of F samples by one wave (lane = hidden unit): each weight read from LDS serves
-// F samples and the F accumulations are independent. Inputs sx[F][XS] (XS >= NIN, a multiple of
-// 4), activations sa[F][kH], outputs sy[F][NOUT]; sx and sa2 may share storage (sx is consumed
-// before sa2 is written). Per output the sum runs over the inputs in ascending order, as in
-// mlpForwardWave.
-template <int NIN, int NOUT, int F, int XS>
-__device__ inline void mlpForwardBatch(const float* net, const float* sx, float* sa1, float* sa2, float* sy, int lane) {
-    using N = NetLds<NIN, NOUT>;
-    static_assert(XS % 4 == 0 && XS >= NIN && NOUT <= 16 && F % 4 == 0, "batch layout");
-    typedef float F4 __attribute__((ext_vector_type(4)));
-    float z[F];
-    {
-        const float* w = net + N::kW1 + lane * N::S1;
-        const float b = net[N::kB1 + lane];
-#pragma unroll
-        for (int f = 0; f < F; ++f) z[f] = b;
-        constexpr int NIN4 = NIN & ~3;
-#pragma unroll 2
-        for (int i = 0; i < NIN4; i += 4) {
-            const float w0 = w[i], w1 = w[i + 1], w2 = w[i + 2], w3 = w[i + 3];
-#pragma unroll
-            for (int f = 0; f < F; ++f) {
-                const F4 x = *reinterpret_cast<const F4*>(sx + f * XS + i);
-                z[f] = fmaf(w3, x[3], fmaf(w2, x[2], fmaf(w1, x[1], fmaf(w0, x[0], z[f]))));
-            }
-        }
-#pragma unroll
-        for (int i = NIN4; i < NIN; ++i) {
-            const float wi = w[i];
-#pragma unroll
-            for (int f = 0; f < F; ++f) z[f] = fmaf(wi, sx[f * XS + i], z[f]);
-        }
-#pragma unroll
-        for (int f = 0; f < F; ++f) sa1[f * kH + lane] = tanhf(z[f]);
-    }
-    waveFence();
-    {
-        const float* w = net + N::kW2 + lane * N::S2;
-        const float b = net[N::kB2 + lane];
-#pragma unroll
-        for (int f = 0; f < F; ++f) z[f] = b;
-#pragma unroll 2
-        for (int k = 0; k < kH; k += 4) {
-            const float w0 = w[k], w1 = w[k + 1], w2 = w[k + 2], w3 = w[k + 3];
-#pragma unroll
-            for (int f = 0; f < F; ++f) {
-                const F4 x = *reinterpret_cast<const F4*>(sa1 + f * kH + k);
-                z[f] = fmaf(w3, x[3], fmaf(w2, x[2], fmaf(w1, x[1], fmaf(w0, x[0], z[f]))));
-            }
-        }
-#pragma unroll
-        for (int f = 0; f < F; ++f) sa2[f * kH + lane] = tanhf(z[f]);
-    }
-    waveFence();
-    {
-        // lane = output j + 16 g: samples g, g + 4, ...
-        const int j = lane & 15, g = lane >> 4;
-        if (j < NOUT) {
-            constexpr int FG = F / 4;
-            const float* w = net + N::kW3 + j * N::S2;
-            const float b = net[N::kB3 + j];
-            float y[FG];
-#pragma unroll
-            for (int c = 0; c < FG; ++c) y[c] = b;
-#pragma unroll 2
-            for (int k = 0; k < kH; k += 4) {
-                const float w0 = w[k], w1 = w[k + 1], w2 = w[k + 2], w3 = w[k + 3];
-#pragma unroll
-                for (int c = 0; c < FG; ++c) {
-                    const F4 x = *reinterpret_cast<const F4*>(sa2 + (g + 4 * c) * kH + k);
-                    y[c] = fmaf(w3, x[3], fmaf(w2, x[2], fmaf(w1, x[1], fmaf(w0, x[0], y[c]))));
-                }
-            }
-#pragma unroll
-            for (int c = 0; c < FG; ++c) sy[(g + 4 * c) * NOUT + j] = y[c];
-        }
-    }
-    waveFence();
-}
-
-// FW faces per wave (4 or 8), kClosureWaves waves per block: the network is staged in LDS
-// once per block and every weight read serves a wave's faces together. With few faces (a 2D
-// truncation boundary) 4 faces per wave spread the work over twice the waves.
-constexpr int kClosureWaves = 4;
-constexpr int kClosureBlock = 64 * kClosureWaves;
-constexpr int kClosureSmall = 4096;  // at most this many faces: 4 faces per wave, else 8
-
-// Exterior states of the learned faces for one stage. Face-node work runs with lane =
-// (face slot, node): 16 lanes per face (NFP <= 16), 4 faces per pass.
-template <int DIM, int P, int NF, typename T, int FW>
+// Exterior states of the learned faces for one stage, 16 faces per block.
+template <int DIM, int P, int NF, typename T>
 __global__ __launch_bounds__(kClosureBlock) void closureKernel(ClosureArgs<T> a) {
     using S = dgk::Sizes<DIM, P>;
     using L = dgk::OpLayout<DIM, P>;
     constexpr int NP = S::NP, NFP = S::NFP, NFC = S::NFC;
-    constexpr int NT = DIM - 1;  // tangential directions
-    constexpr int NIN = DIM * NFP + 2, NOUT = NFP;
-    constexpr int NPASS = FW / 4;
-    static_assert(FW % 4 == 0, "4 faces per pass");
-    constexpr int XS = (NIN + 3) & ~3;
-    static_assert(NFP <= 16 && XS <= kH, "closure lane layout");
-    using N = NetLds<NIN, NOUT>;
-    __shared__ float net[N::kTotal];
-    __shared__ __align__(16) float bufX[kClosureWaves][FW * kH];   // inputs, then second activations
-    __shared__ __align__(16) float bufA[kClosureWaves][FW * kH];   // first activations
-    __shared__ float bufY[kClosureWaves][FW * NOUT];
-    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-    const int slot = lane >> 4, node = lane & 15;
-    const bool nodeLane = node < NFP;
-    const int64_t f0 = static_cast<int64_t>(blockIdx.x) * (kClosureWaves * FW) + wave * FW;
-    // face records of this lane's faces, issued with the network loads
-    int64_t ef[NPASS];
-#pragma unroll
-    for (int ps = 0; ps < NPASS; ++ps) {
-        const int64_t idx = f0 + ps * 4 + slot;
-        ef[ps] = a.faces[idx < a.nfaces ? idx : a.nfaces - 1];
-    }
-    loadNet<NIN, NOUT, kClosureBlock>(a.w, net, tid);
-    __syncthreads();
-    float* sx = bufX[wave];
-    const T c0 = a.ph.c0;
-    // per pass: this lane's face frame and node characteristics
-    T n[NPASS][3], t[NPASS][NT][3], vn0[NPASS], wo[NPASS], wi[NPASS], tt[NPASS][NT], qm[NPASS][NF];
-    float sc[NPASS];
-#pragma unroll
-    for (int ps = 0; ps < NPASS; ++ps) {
-        const int64_t e = ef[ps] / NFC;
-        const int f = static_cast<int>(ef[ps] - e * NFC);
-        n[ps][0] = a.fgeo[(e * NFC + f) * 4];
-        n[ps][1] = a.fgeo[(e * NFC + f) * 4 + 1];
-        n[ps][2] = DIM == 3 ? a.fgeo[(e * NFC + f) * 4 + 2] : T(0);
-        const int nd = a.iops[L::kMask + f * NFP + (nodeLane ? node : 0)];
-        const T* q = a.qin + (e * NP + nd) * NF;
-#pragma unroll
-        for (int k = 0; k < NF; ++k) qm[ps][k] = q[k];
-    }
-#pragma unroll
-    for (int ps = 0; ps < NPASS; ++ps) {
-        T vt0;
-        if constexpr (DIM == 2) {
-            t[ps][0][0] = -n[ps][1];
-            t[ps][0][1] = n[ps][0];
-            t[ps][0][2] = T(0);
-            vn0[ps] = a.ph.v0[0] * n[ps][0] + a.ph.v0[1] * n[ps][1];
-            vt0 = a.ph.v0[0] * t[ps][0][0] + a.ph.v0[1] * t[ps][0][1];
-        } else {
-            vn0[ps] = a.ph.v0[0] * n[ps][0] + a.ph.v0[1] * n[ps][1] + a.ph.v0[2] * n[ps][2];
-            // t1 along the tangential mean flow, else along the axis least aligned with n
-            T u[3];
-            for (int c = 0; c < 3; ++c) u[c] = a.ph.v0[c] - vn0[ps] * n[ps][c];
-            vt0 = sqrt(u[0] * u[0] + u[1] * u[1] + u[2] * u[2]);
-            if (!(vt0 > T(1e-6) * c0)) {
-                const T ax = fabs(n[ps][0]), ay = fabs(n[ps][1]), az = fabs(n[ps][2]);
-                const int k = (ax <= ay && ax <= az) ? 0 : (ay <= az ? 1 : 2);
-                for (int c = 0; c < 3; ++c) u[c] = (c == k ? T(1) : T(0)) - n[ps][k] * n[ps][c];
-                vt0 = T(0);
-            }
-            const T iu = T(1) / sqrt(u[0] * u[0] + u[1] * u[1] + u[2] * u[2]);
-            for (int c = 0; c < 3; ++c) t[ps][0][c] = u[c] * iu;
-            t[ps][1][0] = n[ps][1] * t[ps][0][2] - n[ps][2] * t[ps][0][1];
-            t[ps][1][1] = n[ps][2] * t[ps][0][0] - n[ps][0] * t[ps][0][2];
-            t[ps][1][2] = n[ps][0] * t[ps][0][1] - n[ps][1] * t[ps][0][0];
-        }
-        const T Pv = qm[ps][0] * a.ph.irc0;
-        T Nn = qm[ps][1] * n[ps][0] + qm[ps][2] * n[ps][1];
-        if constexpr (DIM == 3) Nn += qm[ps][3] * n[ps][2];
-        wo[ps] = nodeLane ? Pv + Nn : T(0);
-        wi[ps] = Pv - Nn;
-        for (int c = 0; c < NT; ++c) {
-            T v = qm[ps][1] * t[ps][c][0] + qm[ps][2] * t[ps][c][1];
-            if constexpr (DIM == 3) v += qm[ps][3] * t[ps][c][2];
-            tt[ps][c] = nodeLane ? v : T(0);
-        }
-        // scale: RMS over the face's nodes of the outgoing and tangential characteristics
-        const float wof = static_cast<float>(wo[ps]);
-        float ss = wof * wof;
-        for (int c = 0; c < NT; ++c) {
-            const float ttf = static_cast<float>(tt[ps][c]);
-            ss += ttf * ttf;
-        }
-#pragma unroll
-        for (int off = 8; off > 0; off >>= 1) ss += __shfl_xor(ss, off, 64);
-        sc[ps] = sqrtf(ss / NFP) + 1e-30f;
-        const float is = 1.0f / sc[ps];
-        float* x = sx + (ps * 4 + slot) * XS;
-        if (nodeLane) {
-            x[node] = wof * is;
-            for (int c = 0; c < NT; ++c) x[(1 + c) * NFP + node] = static_cast<float>(tt[ps][c]) * is;
-        } else if (node == NFP) {
-            const float ic0 = static_cast<float>(T(1) / c0);
-            x[DIM * NFP] = static_cast<float>(vn0[ps]) * ic0;
-            x[DIM * NFP + 1] = static_cast<float>(vt0) * ic0;
-        } else if (node == NFP + 1) {
-            for (int i = NIN; i < XS; ++i) x[i] = 0.0f;
-        }
-    }
-    waveFence();
-    mlpForwardBatch<NIN, NOUT, FW, XS>(net, sx, bufA[wave], sx, bufY[wave], lane);
-#pragma unroll
-    for (int ps = 0; ps < NPASS; ++ps) {
-        const int64_t idx = f0 + ps * 4 + slot;
-        if (!nodeLane || idx >= a.nfaces) continue;
-        const T what = static_cast<T>(sc[ps] * bufY[wave][(ps * 4 + slot) * NOUT + node]);
-        const T lam = vn0[ps] - c0;
-        const T wip = (T(2) * lam * what - (lam + c0) * wi[ps]) / (lam - c0);
-        T tp[NT];
-        for (int c = 0; c < NT; ++c)
-            tp[c] = (vn0[ps] >= T(0)) ? tt[ps][c] : -(vn0[ps] + c0) * tt[ps][c] / (vn0[ps] - c0);
-        const T Pp = T(0.5) * (wo[ps] + wip), Np_ = T(0.5) * (wo[ps] - wip);
-        T qp[NF];
-        qp[0] = a.ph.rho0 * c0 * Pp;
-        for (int x = 0; x < DIM; ++x) {
-            T v = Np_ * n[ps][x];
-            for (int c = 0; c < NT; ++c) v += tp[c] * t[ps][c][x];
-            qp[1 + x] = v;
-        }
-        if constexpr (DIM == 2) qp[3] = qm[ps][3];
-        if constexpr (NF == 5) qp[4] = qm[ps][4] + (qp[0] - qm[ps][0]) * a.ph.ic2;
-        T* g = a.ghost + (idx * NFP + node) * NF;
-#pragma unroll
-        for (int k = 0; k < NF; ++k) g[k] = qp[k];
-    }
+    __shared__ __align__(16) ClosureLds lds;
+    const int tid = threadIdx.x, node = tid & 15;
+    const int64_t idx = static_cast<int64_t>(blockIdx.x) * kTileFaces + (tid >> 4);
+    const int64_t ef = a.faces[idx < a.nfaces ? idx : a.nfaces - 1];
+    const ClosureNet w = loadClosureNet(a.w, tid >> 6, tid & 63);
+    const int64_t e = ef / NFC;
+    const int f = static_cast<int>(ef - e * NFC);
+    const T n[3] = {a.fgeo[ef * 4], a.fgeo[ef * 4 + 1], DIM == 3 ? a.fgeo[ef * 4 + 2] : T(0)};
+    const int nd = a.iops[L::kMask + f * NFP + (node < NFP ? node : 0)];
+    T qm[NF], qp[NF];
+    dgk::loadNode<NF>(a.qin + (e * NP + nd) * NF, qm);
+    closureExterior<DIM, NFP, NF>(w, lds, a.ph, n, qm, qp);
+    if (node < NFP && idx < a.nfaces) dgk::storeNode<NF>(a.ghost + (idx * NFP + node) * NF, qp);
 }
 
 // Interior and exterior traces (exterior in the interior element's face-node order) and

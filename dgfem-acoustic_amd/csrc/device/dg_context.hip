@@ -162,7 +162,7 @@ struct dg_context {
     int64_t nLearned = 0;
     int64_t* dLearned = nullptr;
     void* ghost = nullptr;
-    uint16_t* dClosureW = nullptr;
+    dgk::u32x4_t* dClosureW = nullptr;  // the network's matrix-core operands (packClosure)
     int64_t closureParams = 0;
     ClosureFn closureFn = nullptr;
     TraceFn traceFn = nullptr;
@@ -522,17 +522,9 @@ void launchClosure(dg_context* c, const void* qin) {
     a.w = c->dClosureW;
     a.nfaces = c->nLearned;
     a.ph = makePhysics<T>(c->phys);
-    if (c->nLearned <= dgc::kClosureSmall) {
-        constexpr int kPerBlock = dgc::kClosureWaves * 4;
-        const int64_t nb = (c->nLearned + kPerBlock - 1) / kPerBlock;
-        hipLaunchKernelGGL((dgc::closureKernel<DIM, P, NF, T, 4>), dim3(static_cast<unsigned>(nb)),
-                           dim3(dgc::kClosureBlock), 0, c->stream, a);
-    } else {
-        constexpr int kPerBlock = dgc::kClosureWaves * 8;
-        const int64_t nb = (c->nLearned + kPerBlock - 1) / kPerBlock;
-        hipLaunchKernelGGL((dgc::closureKernel<DIM, P, NF, T, 8>), dim3(static_cast<unsigned>(nb)),
-                           dim3(dgc::kClosureBlock), 0, c->stream, a);
-    }
+    const int64_t nb = (c->nLearned + dgc::kTileFaces - 1) / dgc::kTileFaces;
+    hipLaunchKernelGGL((dgc::closureKernel<DIM, P, NF, T>), dim3(static_cast<unsigned>(nb)), dim3(dgc::kClosureBlock), 0,
+                       c->stream, a);
 }
 
 template <int DIM, int P, int NF, typename T>
@@ -1359,8 +1351,8 @@ dg_status dg_create(const dg_mesh_desc* m, const dg_physics* ph, const dg_option
             c->dLearned = uploadVec(c, c->mesh.learnedFaces);
             c->ghost = alloc(static_cast<size_t>(c->nLearned) * c->Nfp * c->nf);
             c->closureParams = dgc::numParams(c->dim * c->Nfp + 2, c->Nfp);
-            c->dClosureW = devAlloc<uint16_t>(c, c->closureParams);
-            HIPCHK(hipMemset(c->dClosureW, 0, c->closureParams * sizeof(uint16_t)));
+            c->dClosureW = devAlloc<dgk::u32x4_t>(c, dgc::kNetWords);
+            HIPCHK(hipMemset(c->dClosureW, 0, dgc::kNetWords * sizeof(dgk::u32x4_t)));
         }
         c->resPartial = devAlloc<double>(c, static_cast<size_t>(c->nblocks) * 5);
         HIPCHK(hipMemset(c->resPartial, 0, static_cast<size_t>(c->nblocks) * 5 * sizeof(double)));
@@ -1401,7 +1393,9 @@ dg_status dg_set_closure(dg_context* c, const uint16_t* params, int64_t n) {
     try {
         HIPCHK(hipSetDevice(c->device));
         HIPCHK(hipStreamSynchronize(c->stream));
-        HIPCHK(hipMemcpy(c->dClosureW, params, n * sizeof(uint16_t), hipMemcpyHostToDevice));
+        std::vector<uint32_t> words(dgc::kNetWords * 4, 0);
+        dgc::packClosure(c->dim * c->Nfp + 2, c->Nfp, params, words.data());
+        HIPCHK(hipMemcpy(c->dClosureW, words.data(), words.size() * sizeof(uint32_t), hipMemcpyHostToDevice));
     } catch (const std::exception& ex) {
         return fail(c, DG_ERR_DEVICE, ex.what());
     }
