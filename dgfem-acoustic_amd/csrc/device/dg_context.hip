@@ -128,7 +128,7 @@ struct dg_context {
     uint8_t* hVF = nullptr;
     bool tablesDirty = true;
     // resident time loop (0 blocks: not used for this grid)
-    int64_t resBlocks = 0;
+    int64_t resBlocks = 0, resGrid = 0;  // blocks of elements; with those of learned faces
     int resShape = 0;                  // dgk::kRes*
     int resChunk = 0;                  // steps per launch
     unsigned char* resMail = nullptr;  // two sets of mailboxes, then outcomes and counts per chunk
@@ -1000,12 +1000,11 @@ void captureGraphs(dg_context* c, int integrator, bool resid, int steps) {
 }
 
 // Grids that run in the resident time loop (dg_resident.hpp): at most as many 256-thread blocks as
-// the chip holds at once, on meshes without learned faces (their exterior states come from a kernel
-// of their own before every stage) and without an explicit DGFEM_KERNEL or DGFEM_POST_BRANCH (both
-// ask for launches per stage). DGFEM_RESIDENT=0 switches it off.
+// the chip holds at once, without an explicit DGFEM_KERNEL or DGFEM_POST_BRANCH (both ask for
+// launches per stage). DGFEM_RESIDENT=0 switches it off.
 void pickResident(dg_context* c) {
     const char* env = std::getenv("DGFEM_RESIDENT");
-    if (c->nLearned > 0 || (env && env[0] == '0')) return;
+    if (env && env[0] == '0') return;
     for (const char* name : {"DGFEM_KERNEL", "DGFEM_POST_BRANCH"}) {
         const char* v = std::getenv(name);
         if (v && v[0]) return;
@@ -1021,14 +1020,15 @@ void pickResident(dg_context* c) {
         if (eb == 0) return;
         n = (c->K + eb - 1) / eb;
         c->resShape = shape;
-        if (n <= static_cast<int64_t>(cus) * dgk::residentBlocksPerCu(c->dim, c->p, c->nf, c->precision == DG_FP64, shape)) {
+        c->resGrid = n + (c->nLearned + dgc::kTileFaces - 1) / dgc::kTileFaces;
+        if (c->resGrid <= static_cast<int64_t>(cus) * dgk::residentBlocksPerCu(c->dim, c->p, c->nf, c->precision == DG_FP64, shape)) {
             c->resBlocks = n;
             break;
         }
     }
     if (c->resBlocks == 0) return;
     const size_t chunks = c->ringSlots / kResMinChunk, partials = static_cast<size_t>(kResMaxChunk) * n * 5;
-    c->resMailBytes = align256(static_cast<size_t>(c->K) * c->Nfc * c->Nfp * c->nf * c->tsize);
+    c->resMailBytes = align256((static_cast<size_t>(c->K) * c->Nfc + c->nLearned) * c->Nfp * c->nf * c->tsize);
     c->resMail = devAlloc<unsigned char>(c, 2 * c->resMailBytes + partials * 8 + 2 * chunks * sizeof(int));
     c->resSteps = reinterpret_cast<double*>(c->resMail + 2 * c->resMailBytes);
     c->resOutcome = reinterpret_cast<int*>(c->resSteps + partials);
@@ -1043,6 +1043,10 @@ hipError_t launchChunk(dg_context* c, int chunk, int64_t slot0, int steps, int64
     a.snap = resid ? static_cast<const T*>(c->snap) : nullptr;
     a.mail = reinterpret_cast<T*>(c->resMail);
     a.mailBytes = static_cast<int>(c->resMailBytes);
+    a.learned = c->dLearned;
+    a.nLearned = static_cast<int>(c->nLearned);
+    a.net = c->dClosureW;
+    a.blocks = static_cast<int>(c->resBlocks);
     a.geo = static_cast<const T*>(c->geo);
     a.fgeo = static_cast<const T*>(c->fgeo);
     a.nbr = c->nbr;
@@ -1068,7 +1072,7 @@ hipError_t launchChunk(dg_context* c, int chunk, int64_t slot0, int steps, int64
     a.slots = c->nseg * 256;
     a.euler = integrator == DG_EULER;
     a.ph = makePhysics<T>(c->phys);
-    return dgk::launchResident<T>(c->dim, c->p, c->nf, c->resShape, a, sourceArgs(c), static_cast<unsigned>(c->resBlocks), c->stream);
+    return dgk::launchResident<T>(c->dim, c->p, c->nf, c->resShape, a, sourceArgs(c), static_cast<unsigned>(c->resGrid), c->stream);
 }
 
 // Enqueues a batch of n steps (state, step tables and counters set) in the resident time loop;

@@ -48,7 +48,8 @@ const void* kernelOf(int dim, int p, int nf, int shape) {
         };
         f = shape == kResRows     ? of(std::integral_constant<int, kResRows>{})
             : shape == kResSpread ? of(std::integral_constant<int, kResSpread>{})
-                                  : of(std::integral_constant<int, kResDense>{});
+            : shape == kResDense  ? of(std::integral_constant<int, kResDense>{})
+                                  : of(std::integral_constant<int, kResTight>{});
         return true;
     });
     return f;
@@ -60,7 +61,7 @@ int residentElements(int dim, int p, int shape) {
     int eb = 0;
     dispatch(dim, p, 4, [&](auto dc, auto pc, auto) {
         constexpr int D = decltype(dc)::value, P = decltype(pc)::value;
-        eb = shape == kResDense ? ResidentShape<D, P, 4, float, kResDense>::EB : ResidentShape<D, P, 4, float, kResSpread>::EB;
+        eb = shape >= kResDense ? ResidentShape<D, P, 4, float, kResDense>::EB : ResidentShape<D, P, 4, float, kResSpread>::EB;
         return true;
     });
     return eb;
@@ -69,8 +70,14 @@ int residentElements(int dim, int p, int shape) {
 int residentBlocksPerCu(int dim, int p, int nf, bool fp64, int shape) {
     const void* f = fp64 ? kernelOf<double>(dim, p, nf, shape) : kernelOf<float>(dim, p, nf, shape);
     int n = 0;
-    if (!f || hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, f, kBlock, 0) != hipSuccess) return 0;
-    return n;
+    hipFuncAttributes attr{};
+    if (!f || hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, f, kBlock, 0) != hipSuccess ||
+        hipFuncGetAttributes(&attr, f) != hipSuccess)
+        return 0;
+    // the LDS of a block is allocated in units the occupancy query does not round to: 5 blocks of
+    // 32,504 bytes fit the 160 KB of a CU by division but were not resident together
+    const int lds = (160 * 1024) / (static_cast<int>(attr.sharedSizeBytes) + 2048);
+    return n < lds ? n : lds;
 }
 
 template <typename T>

@@ -16,6 +16,12 @@
 // of the same face node; the owner writes the same mailbox two epochs later, after it received
 // that trace, so a mailbox is always empty when it is written.
 //
+// Learned faces (DG_BC_LEARNED): further blocks of the launch evaluate the closure network for 16
+// faces each. To the block that owns such a face they are one more neighbour: they receive its trace
+// in an inbox and answer into the mailboxes of its face nodes. (Evaluated by the owning block itself
+// the network's registers came on top of the block's state: its spills made 1,000-block grids slower
+// than a launch per stage.)
+//
 // The blocks wait for one another, so the launch is cooperative (all blocks resident, or it
 // fails). Every wait is bounded by a clock all the same (it also ends where a state contains the
 // kEmpty pattern): a thread that waits too long sets the chunk's outcome to kAborted, every block
@@ -25,12 +31,13 @@
 // Residual partials and the state at observer nodes are stored per step and reduced after the
 // chunk by residentPostKernel, in the order of postKernel.
 #pragma once
+#include "dg_closure.hpp"
 #include "dg_kernels.hpp"
 
 namespace dgk {
 
 enum : int { kPending = 0, kDone = 1, kAborted = 2 };
-enum : int { kResRows = 0, kResSpread = 1, kResDense = 2, kResShapes = 3 };
+enum : int { kResRows = 0, kResSpread = 1, kResDense = 2, kResTight = 3, kResShapes = 4 };
 
 constexpr uint32_t kEmpty = 0xffffffffu;
 
@@ -39,8 +46,13 @@ struct ResidentArgs {
     T* __restrict__ u;
     T* __restrict__ ulo;
     const T* __restrict__ snap;  // residual snapshot, or null without residuals
-    T* mail;                     // two sets of mailboxes [K][NFT] of NF values, empty at the start of a
-    int mailBytes;               //   chunk, and the bytes of one set
+    T* mail;                     // two sets of mailboxes of NF values, [K][NFT] for the face nodes, then
+    int mailBytes;               //   [learned faces][NFP] inboxes; empty at the start of a chunk; and the
+                                 //   bytes of one set
+    const int64_t* __restrict__ learned;  // the learned faces (element * NFC + face),
+    int nLearned;                         //   their number and the network (packClosure)
+    const u32x4_t* __restrict__ net;
+    int blocks;                           // blocks of elements; the others evaluate learned faces
     const T* __restrict__ geo;
     const T* __restrict__ fgeo;
     const int32_t* __restrict__ nbr;
@@ -73,27 +85,31 @@ struct ResidentArgs {
 //     256), which shortens the chain of a stage: 2 blocks per CU;
 //   kResSpread: the same elements per block, operators in LDS: 4 blocks per CU (FP64 tetrahedra and
 //     order 1: 3);
-//   kResDense: as many elements as have their nodes covered, several face nodes per thread.
+//   kResDense: as many elements as have their nodes covered, several face nodes per thread;
+//   kResTight: the same in FP32 at 5 blocks per CU.
 // Measured against a launch per stage (us per step, 4 fields, one observer; start > resident):
 //   triangles p=3 mixed: 200 elements 24.4 > 8.6, 8,000 26.6 > 9.6, 18,000 28.8 > 13.7;
 //   FP64 26.5 > 10.5, 31.5 > 14.4, 38.6 > 23.7; p=1 mixed 40,000 25.8 > 12.8;
 //   tetrahedra p=2 mixed: 160 29.0 > 10.4, 4,400 29.6 > 11.3; FP64 32.1 > 15.2, 33.5 > 18.6;
-//   p=3 mixed: 8,000 38.0 > 24.1, FP64 54.3 > 41.3.
+//   p=3 mixed: 8,000 38.0 > 24.1, FP64 54.3 > 41.3;
+//   learned walls: triangles p=4 mixed 200 42.0 > 19.6, 20,000 54.7 > 26.5; tetrahedra p=3 mixed
+//   160 45.6 > 22.7, 8,000 56.7 > 29.4.
 template <int DIM, int P, int NF, typename T, int SHAPE>
 struct ResidentShape {
     using S = Sizes<DIM, P>;
     static constexpr bool kFp64 = sizeof(T) == 8;
-    static constexpr int EB = kBlock / (SHAPE != kResDense && S::NFT > S::NP ? S::NFT : S::NP);
+    static constexpr int EB = kBlock / (SHAPE < kResDense && S::NFT > S::NP ? S::NFT : S::NP);
     static constexpr int kFIt = (EB * S::NFT + kBlock - 1) / kBlock;  // face nodes per thread
     static constexpr int kRowRegs = (S::NP * DIM + S::NFT) * static_cast<int>(sizeof(T)) / 4;
     static constexpr bool kOpsReg = SHAPE == kResRows && kRowRegs <= (!kFp64 ? 96 : NF == 4 ? 64 : 44);
     // waves per SIMD asked for: bounds the registers so that this many blocks stay on a CU
-    static constexpr int kWaves = SHAPE == kResRows ? 2 : kFp64 && (SHAPE == kResDense || DIM == 3 || P == 1) ? 3 : 4;
+    static constexpr int kWaves = SHAPE == kResRows ? 2 : kFp64 && (SHAPE == kResDense || DIM == 3 || P == 1) ? 3 : SHAPE == kResTight ? 5 : 4;
     // Not built where it lost to a launch per stage, its registers spilled: dense blocks with three
     // face nodes per thread (tetrahedra p=2, 13,000 elements, FP64: 47 against 45 us per step, 5
     // fields 82 against 57) or of FP64 triangles of order 1, and spread ones of 5 FP64 fields on
     // tetrahedra of order 1 (13,000 elements: 72 against 34)
     static constexpr bool kBuilt = SHAPE == kResDense    ? kFIt <= 2 && !(kFp64 && P == 1)
+                                   : SHAPE == kResTight  ? kFIt <= 2 && !kFp64
                                    : SHAPE == kResSpread ? !(kFp64 && DIM == 3 && P == 1 && NF == 5)
                                                          : true;
 };
@@ -204,8 +220,11 @@ __global__ __launch_bounds__(kBlock, (ResidentShape<DIM, P, NF, T, SHAPE>::kWave
     constexpr int QS = ldsStride(NP * NF), FS = ldsStride(NFT * NF);
     constexpr int kOpsN = R::kOpsReg ? 1 : L::kN;  // Dw and LIFT; FP64 as two 32-bit planes (see stageKernel)
     constexpr bool kPlanes = sizeof(T) == 8;
-    __shared__ __align__(32) T sQ[EB * QS];
-    __shared__ __align__(32) T sF[EB * FS];
+    // the stage input and the scaled fluxes of the elements, or the network's exchange
+    constexpr int kQF = EB * (QS + FS), kNetLds = static_cast<int>(sizeof(dgc::ClosureLds) / sizeof(T));
+    __shared__ __align__(32) T sQF[kQF > kNetLds ? kQF : kNetLds];
+    T* const sQ = sQF;
+    T* const sF = sQF + EB * QS;
     __shared__ T sJ[EB * JJ];
     __shared__ __align__(32) T sN[EB * NFC * 8];  // unit normal, Fscale; h n, h (v0.n) with h = Fscale / 2
     __shared__ __align__(16) T sOps[kOpsN];
@@ -217,16 +236,64 @@ __global__ __launch_bounds__(kBlock, (ResidentShape<DIM, P, NF, T, SHAPE>::kWave
         return;
     }
     const int tid = threadIdx.x;
-    const int nblk = static_cast<int>(gridDim.x);
-    const int bi = static_cast<int>(xcdRemap(blockIdx.x, gridDim.x));
+    int* const outcome = &a.outcome[a.chunk];
+    const __amdgpu_buffer_rsrc_t mail = mailBuffer(a.mail, 2 * a.mailBytes);
+    const int inbox0 = static_cast<int>(a.K) * NFT;
+    const int fifth = (inbox0 + a.nLearned * NFP) * 4 * static_cast<int>(sizeof(T));
+    T none[NF];
+#pragma unroll
+    for (int k = 0; k < NF; ++k) none[k] = emptyValue<T>();
+    const int nst = a.euler ? 1 : 4;
+    if (tid == 0) sAbort = 0;
+
+    if (static_cast<int>(blockIdx.x) >= a.blocks) {
+        // ---- a block of learned faces: trace in, exterior state out, once per stage ----
+        if constexpr (DIM == 2 || P <= 3) {
+            dgc::ClosureLds& lds = *reinterpret_cast<dgc::ClosureLds*>(sQF);
+            const int node = tid & 15, idx = (static_cast<int>(blockIdx.x) - a.blocks) * dgc::kTileFaces + (tid >> 4);
+            const bool mine = idx < a.nLearned && node < NFP;
+            const int lf = idx < a.nLearned ? idx : a.nLearned - 1;
+            const int64_t ef = a.learned[lf];
+            const int fa = static_cast<int>(ef % NFC) * NFP + (node < NFP ? node : 0);
+            const int in = inbox0 + lf * NFP + (node < NFP ? node : 0), out = static_cast<int>(ef / NFC) * NFT + fa;
+            const T n[3] = {a.fgeo[ef * 4], a.fgeo[ef * 4 + 1], DIM == 3 ? a.fgeo[ef * 4 + 2] : T(0)};
+            const dgc::ClosureNet w = dgc::loadClosureNet(a.net, tid >> 6, tid & 63);
+            __syncthreads();
+            for (int epoch = 0; epoch < a.steps * nst; ++epoch) {
+                T qm[NF], qp[NF];
+                const int set = (epoch & 1) * a.mailBytes;
+                if (mine) {
+                    loadMail<NF>(mail, set, fifth, in, qm);
+                    const uint64_t t0 = __builtin_amdgcn_s_memrealtime();
+                    for (int tries = 1; !arrived<NF>(qm); ++tries) {
+                        if ((tries % 64 == 0 || a.patience == 0) && giveUp(outcome, t0, a.patience)) {
+                            sAbort = 1;
+                            break;
+                        }
+                        loadMail<NF>(mail, set, fifth, in, qm);
+                    }
+                    storeMail<NF>(mail, set, fifth, in, none);
+                } else {
+#pragma unroll
+                    for (int k = 0; k < NF; ++k) qm[k] = T(0);
+                }
+                dgc::closureExterior<DIM, NFP, NF>(w, lds, a.ph, n, qm, qp);
+                if (sAbort) return;  // (set before the barriers inside)
+                waitStores();
+                if (mine) storeMail<NF>(mail, set, fifth, out, qp);
+            }
+        }
+        return;
+    }
+
+    const int nblk = a.blocks;
+    const int bi = static_cast<int>(xcdRemap(blockIdx.x, nblk));
     const int64_t e0 = static_cast<int64_t>(bi) * EB;
     const int nE = static_cast<int>((a.K - e0) < EB ? (a.K - e0) : EB);
     const bool active = tid < nE * NP;
     const int el = active ? tid / NP : 0, i = active ? tid - el * NP : 0;
     const int64_t base = (e0 * NP + (active ? tid : 0)) * NF;
-    int* const outcome = &a.outcome[a.chunk];
     uint32_t* const sOpsW = reinterpret_cast<uint32_t*>(sOps);
-    if (tid == 0) sAbort = 0;
 
     // ---- once per chunk: state, geometry, operators, the addresses of this thread's face nodes ----
     T u[NF], ulo[NF], acc[NF], q[NF];
@@ -301,6 +368,10 @@ __global__ __launch_bounds__(kBlock, (ResidentShape<DIM, P, NF, T, SHAPE>::kWave
                 fExt[c] = local ? static_cast<int>(lb) * QS + a.iops[L::kMask + opp] * NF
                                 : static_cast<int>(e0 + fe) * NFT + fa;
                 fSend[c] = nb * NFT + opp;
+            } else if (nb <= -3) {  // learned: the block that evaluates face -3 - nb
+                fKind[c] = kRemote;
+                fExt[c] = static_cast<int>(e0 + fe) * NFT + fa;
+                fSend[c] = inbox0 + (-3 - nb) * NFP + an;
             } else {
                 fKind[c] = nb == -2 ? kReflect : kAbsorb;
             }
@@ -329,11 +400,6 @@ __global__ __launch_bounds__(kBlock, (ResidentShape<DIM, P, NF, T, SHAPE>::kWave
             srcCount = static_cast<int>(s.coverOff[lo + 1]) - srcFirst;
         }
     }
-    const __amdgpu_buffer_rsrc_t mail = mailBuffer(a.mail, 2 * a.mailBytes);
-    const int fifth = static_cast<int>(a.K) * NFT * 4 * static_cast<int>(sizeof(T));
-    T none[NF];
-#pragma unroll
-    for (int k = 0; k < NF; ++k) none[k] = emptyValue<T>();
     T qm[kFIt][NF];  // this thread's face nodes: own values of the current stage input
     auto sendTraces = [&](int epoch) __attribute__((always_inline)) {
 #pragma unroll
@@ -348,7 +414,6 @@ __global__ __launch_bounds__(kBlock, (ResidentShape<DIM, P, NF, T, SHAPE>::kWave
     __syncthreads();
     sendTraces(epoch);
 
-    const int nst = a.euler ? 1 : 4;
     int pendingStep = -1;  // step whose residual rows in sRed are still to be summed
     for (int step = 0; step < a.steps; ++step) {
         const int64_t slot = a.slot0 + step;

@@ -20,7 +20,8 @@ RHO0, C0 = 1.225, 340.0
 TOL = {dg.DG_MIXED: 3e-6, dg.DG_FP64: 6e-15 * 2}
 
 
-def _run(m, bc, order, fields, precision, resident, monkeypatch, integrator=dg.DG_RK4, steps=50, save=17, patience=None):
+def _run(m, bc, order, fields, precision, resident, monkeypatch, integrator=dg.DG_RK4, steps=50, save=17, patience=None,
+         net=None):
     monkeypatch.setenv("DGFEM_RESIDENT", resident)
     if patience is not None:
         monkeypatch.setenv("DGFEM_RESIDENT_PATIENCE", patience)
@@ -28,6 +29,8 @@ def _run(m, bc, order, fields, precision, resident, monkeypatch, integrator=dg.D
     s = dg.Solver(m.node_coords, m.element_vertices, order, bc, v0=(30.0, -20.0, 10.0 if dim == 3 else 0.0), rho0=RHO0,
                   c0=C0, fields=dg.DG_FIELDS_LEE5 if fields == 5 else dg.DG_FIELDS_REF4, precision=precision,
                   steps_per_graph=8)
+    if net is not None:
+        s.set_closure(net)
     X = m.node_coords.reshape(-1, 3)
     u = np.zeros(s.state_shape)
     u[0] = np.exp(-((X - 0.2 * np.array([1, 1, dim - 2])) ** 2).sum(1) / 0.1)
@@ -72,6 +75,22 @@ def test_resident_equals_launch_per_stage(dim, order, fields, n, precision, monk
     bc = dg.resolve_bc_sides(m, [(0x3, dg.DG_BC_REFLECTING), (0x3C if dim == 3 else 0xC, dg.DG_BC_ABSORBING)])
     args = (m, bc, order, fields, precision)
     _close(_run(*args, "1", monkeypatch), _run(*args, "0", monkeypatch), TOL[precision])
+
+
+@pytest.mark.parametrize("dim,order,fields,n", [(2, 1, 5, 2), (2, 1, 4, 100), (2, 2, 4, 90), (2, 3, 5, 9), (2, 3, 4, 95),
+                                                (2, 4, 4, 100), (2, 5, 4, 40), (3, 1, 4, 9), (3, 2, 5, 3), (3, 3, 4, 2),
+                                                (3, 3, 4, 11)])
+@pytest.mark.parametrize("precision", [dg.DG_FP64, dg.DG_MIXED])
+def test_resident_learned_faces(dim, order, fields, n, precision, monkeypatch):
+    """Learned faces on all but one pair of sides, evaluated by blocks of their own; the network is
+    FP32 in both precisions."""
+    print(f"case resident learned dim={dim} order={order} fields={fields} n={n} precision={precision}", flush=True)
+    m = dg.box_mesh(dim, n, order, jitter=0.1, seed=n)
+    bc = dg.resolve_bc_sides(m, [(0x3, dg.DG_BC_REFLECTING), (0x3C if dim == 3 else 0xC, dg.DG_BC_LEARNED)])
+    nfp = order + 1 if dim == 2 else dg.num_nodes(2, order)
+    net = dg.to_bf16(dg.closure_init(nfp, seed=4, out_scale=0.1, dim=dim))
+    args = (m, bc, order, fields, precision)
+    _close(_run(*args, "1", monkeypatch, net=net), _run(*args, "0", monkeypatch, net=net), TOL[dg.DG_MIXED])
 
 
 @pytest.mark.parametrize("dim,order,n", [(2, 2, 20), (3, 2, 5)])
