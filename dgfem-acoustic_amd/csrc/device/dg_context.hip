@@ -23,6 +23,7 @@
 #include "dg_kernels.hpp"
 #include "dg_kernels_bf16.hpp"
 #include "dg_resident.hpp"
+#include "dg_stage_quad.hpp"
 
 namespace {
 
@@ -101,8 +102,12 @@ struct dg_context {
     int32_t *nbr = nullptr, *iops = nullptr;
     uint8_t *code = nullptr, *toCanon = nullptr;
     double* resPartial = nullptr;
-    double* resGroup = nullptr;  // per-group residual sums when nblocks > 4 kResGroup
+    double* resGroup = nullptr;  // per-group residual sums when nPartials > 4 kResGroup
     int64_t nblocks = 0, nResGroups = 0;
+    int64_t nPartials = 0;       // residual partials per step: blocks of the stage launch
+    float* fgeoH = nullptr;      // (mixed; quad and resident kernels) per face h n, h (v0.n), h = Fscale / 2
+    void* quadFrag = nullptr;    // operator of the lane-per-field stage kernel, or null: not used
+    int64_t quadGrid[5] = {0, 0, 0, 0, 0};  // its blocks per mode (kMode*)
     // sources / observers (host definitions + device tables)
     std::vector<std::vector<int64_t>> srcNodes;
     std::vector<std::array<double, 5>> srcParams;  // kind, amp, freq, phase, duration
@@ -485,10 +490,10 @@ void launchPost(dg_context* c) {
     hipStream_t st = c->postStream ? c->postStream : c->stream;
     dgk::PostArgs p{};
     p.resPartial = c->resPartial;
-    p.nblocks = c->nblocks;
+    p.nblocks = c->nPartials;
     if (c->resGroup && c->curResid) {
         hipLaunchKernelGGL(dgk::residualGroupKernel, dim3(static_cast<unsigned>(c->nResGroups)), dim3(256), 0, st,
-                           static_cast<const double*>(c->resPartial), c->nblocks, c->resGroup);
+                           static_cast<const double*>(c->resPartial), c->nPartials, c->resGroup);
         p.resPartial = c->resGroup;
         p.nblocks = c->nResGroups;
     }
@@ -708,7 +713,16 @@ bool pickP(dg_context* c) {
 // One stage: exterior states of the learned faces from the stage input, then the stage.
 void runStage(dg_context* c, int stage, const void* qin, void* qout, void* uout, bool snap) {
     if (c->nLearned > 0) c->closureFn(c, qin);
-    c->stageFn(c, stage, qin, qout, uout, snap);
+    if (c->quadFrag) {
+        dgk::StageArgs<float> a = stageArgs<float, true>(c, stage, qin, qout, uout, snap);
+        a.vfrag = static_cast<const float*>(c->quadFrag);
+        a.fgeo = c->fgeoH;
+        const int mode = dgk::stageMode(stage);
+        dgk::launchStageQuad(mode, a, (c->K + dgk::kQuadGroup - 1) / dgk::kQuadGroup,
+                             static_cast<unsigned>(c->quadGrid[mode]), c->stream);
+    } else {
+        c->stageFn(c, stage, qin, qout, uout, snap);
+    }
 }
 
 bool pickKernels(dg_context* c) {
@@ -999,6 +1013,32 @@ void captureGraphs(dg_context* c, int integrator, bool resid, int steps) {
     c->gResid = resid ? 1 : 0;
 }
 
+// Grids whose stages run with a lane per (element, field) (dg_kernels_quad.hpp) in place of the
+// variant that dg_get_info names: mixed-precision tetrahedra of order 3 with 4 fields, from the
+// size on where its persistent waves have several groups of elements each (us per step, vm and
+// this: 48,000 elements 114 and 114, 82,944 169 and 169, 131,712 247 and 250, 196,608 367 and 330,
+// 413,526 753 and 676; with learned walls 82,944 189 and 193, 196,608 389 and 363).
+// DGFEM_QUAD = 0 | 1 overrides the size.
+constexpr int64_t kQuadMinElements = 163840;
+
+void pickQuad(dg_context* c, const dg::RefElement& R) {
+    const char* kernel = std::getenv("DGFEM_KERNEL");
+    const char* env = std::getenv("DGFEM_QUAD");
+    if (c->precision != DG_MIXED || c->nf != 4 || (kernel && kernel[0])) return;
+    if (env && env[0] == '0') return;
+    if (!(env && env[0] == '1') && c->K < kQuadMinElements) return;
+    if (c->K * c->Np * 16 >= (int64_t(1) << 32)) return;  // the kernel's gathers use 32-bit byte offsets
+    std::vector<double> frag;
+    if (!dgk::buildQuadFrag(c->dim, c->p, R.Dw.data(), R.LIFT.data(), R.fmask.data(), frag)) return;
+    int cus = 0;
+    HIPCHK(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, c->device));
+    c->quadFrag = devAlloc<float>(c, frag.size());
+    uploadAs<float>(c, c->quadFrag, frag);
+    for (int mode = 0; mode < 5; ++mode)
+        c->quadGrid[mode] = std::min<int64_t>((c->K + dgk::kQuadPerBlock - 1) / dgk::kQuadPerBlock,
+                                              static_cast<int64_t>(cus) * dgk::quadBlocksPerCu(mode));
+}
+
 // Grids that run in the resident time loop (dg_resident.hpp): at most as many 256-thread blocks as
 // the chip holds at once, without an explicit DGFEM_KERNEL or DGFEM_POST_BRANCH (both ask for
 // launches per stage). DGFEM_RESIDENT=0 switches it off.
@@ -1049,6 +1089,8 @@ hipError_t launchChunk(dg_context* c, int chunk, int64_t slot0, int steps, int64
     a.blocks = static_cast<int>(c->resBlocks);
     a.geo = static_cast<const T*>(c->geo);
     a.fgeo = static_cast<const T*>(c->fgeo);
+    a.fgeoH = c->fgeoH;
+    if (sizeof(T) == 4 && !a.fgeoH) return hipErrorInvalidValue;
     a.nbr = c->nbr;
     a.code = c->code;
     a.ops = static_cast<const T*>(c->ops);
@@ -1172,7 +1214,8 @@ void destroyContext(dg_context* c) {
     if (c->device >= 0) (void)hipSetDevice(c->device);
     releaseGraphs(c);
     freeTables(c);
-    for (void* p : {c->u, c->ulo, c->qa, c->snap, c->geo, c->fgeo, c->ops, c->afrag, c->afragBf})  // qa: with acc, qb
+    for (void* p : {c->u, c->ulo, c->qa, c->snap, c->geo, c->fgeo, c->ops, c->afrag, c->afragBf,
+                    c->quadFrag, static_cast<void*>(c->fgeoH)})  // qa: with acc, qb
         devFree(p);
     devFree(c->nbr);
     devFree(c->iops);
@@ -1358,10 +1401,12 @@ dg_status dg_create(const dg_mesh_desc* m, const dg_physics* ph, const dg_option
             c->dClosureW = devAlloc<dgk::u32x4_t>(c, dgc::kNetWords);
             HIPCHK(hipMemset(c->dClosureW, 0, dgc::kNetWords * sizeof(dgk::u32x4_t)));
         }
-        c->resPartial = devAlloc<double>(c, static_cast<size_t>(c->nblocks) * 5);
-        HIPCHK(hipMemset(c->resPartial, 0, static_cast<size_t>(c->nblocks) * 5 * sizeof(double)));
-        if (c->nblocks > 4 * dgk::kResGroup) {  // below that the extra launch costs what it saves
-            c->nResGroups = (c->nblocks + dgk::kResGroup - 1) / dgk::kResGroup;
+        pickQuad(c, R);
+        c->nPartials = c->quadFrag ? std::max(c->quadGrid[dgk::kModeFinal], c->quadGrid[dgk::kModeEuler]) : c->nblocks;
+        c->resPartial = devAlloc<double>(c, static_cast<size_t>(c->nPartials) * 5);
+        HIPCHK(hipMemset(c->resPartial, 0, static_cast<size_t>(c->nPartials) * 5 * sizeof(double)));
+        if (c->nPartials > 4 * dgk::kResGroup) {  // below that the extra launch costs what it saves
+            c->nResGroups = (c->nPartials + dgk::kResGroup - 1) / dgk::kResGroup;
             c->resGroup = devAlloc<double>(c, static_cast<size_t>(c->nResGroups) * 5);
         }
         c->ringSlots = 4096;
@@ -1373,6 +1418,21 @@ dg_status dg_create(const dg_mesh_desc* m, const dg_physics* ph, const dg_option
         HIPCHK(hipHostMalloc(reinterpret_cast<void**>(&c->hT), sizeof(double) * c->ringSlots));
         HIPCHK(hipHostMalloc(reinterpret_cast<void**>(&c->hRes), sizeof(double) * c->ringSlots * 5));
         pickResident(c);
+        if (c->precision == DG_MIXED && (c->quadFrag || c->resBlocks > 0)) {
+            // the interior flux's coefficients rounded once from FP64
+            std::vector<double> fh(fgeo.size());
+            for (size_t x = 0; x < fgeo.size(); x += 4) {
+                const double h = 0.5 * fgeo[x + 3];
+                double hv = 0.0;
+                for (int q = 0; q < 3; ++q) {
+                    fh[x + q] = h * fgeo[x + q];
+                    hv += c->phys.v0[q] * fh[x + q];
+                }
+                fh[x + 3] = hv;
+            }
+            c->fgeoH = devAlloc<float>(c, fh.size());
+            uploadAs<float>(c, c->fgeoH, fh);
+        }
         c->tablesDirty = true;
         syncTables(c);
         HIPCHK(hipDeviceSynchronize());
