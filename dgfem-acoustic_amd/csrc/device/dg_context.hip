@@ -23,6 +23,7 @@
 #include "dg_kernels.hpp"
 #include "dg_kernels_bf16.hpp"
 #include "dg_resident.hpp"
+#include "dg_stage_f64.hpp"
 #include "dg_stage_quad.hpp"
 
 namespace {
@@ -107,6 +108,8 @@ struct dg_context {
     int64_t nPartials = 0;       // residual partials per step: blocks of the stage launch
     float* fgeoH = nullptr;      // (mixed; quad and resident kernels) per face h n, h (v0.n), h = Fscale / 2
     void* quadFrag = nullptr;    // operator of the lane-per-field stage kernel, or null: not used
+    double* f64Frag = nullptr;   // operator of the FP64 matrix-core stage kernel, or null: not used
+    int64_t f64Grid = 0;         // its blocks
     int64_t quadGrid[5] = {0, 0, 0, 0, 0};  // its blocks per mode (kMode*)
     // sources / observers (host definitions + device tables)
     std::vector<std::vector<int64_t>> srcNodes;
@@ -720,6 +723,11 @@ void runStage(dg_context* c, int stage, const void* qin, void* qout, void* uout,
         const int mode = dgk::stageMode(stage);
         dgk::launchStageQuad(mode, a, (c->K + dgk::kQuadGroup - 1) / dgk::kQuadGroup,
                              static_cast<unsigned>(c->quadGrid[mode]), c->stream);
+    } else if (c->f64Frag) {
+        dgk::StageArgs<double> a = stageArgs<double, false>(c, stage, qin, qout, uout, snap);
+        a.vfrag = c->f64Frag;
+        dgk::launchStageF64(c->p, c->nf, dgk::stageMode(stage), a,
+                            static_cast<unsigned>(c->f64Grid), c->stream);
     } else {
         c->stageFn(c, stage, qin, qout, uout, snap);
     }
@@ -1039,6 +1047,26 @@ void pickQuad(dg_context* c, const dg::RefElement& R) {
                                               static_cast<int64_t>(cus) * dgk::quadBlocksPerCu(mode));
 }
 
+// Grids that take the FP64 matrix-core stage kernel (dg_kernels_f64.hpp): tetrahedra of order 4 and
+// 5, without an explicit DGFEM_KERNEL. Its blocks take 16 elements, so a small grid leaves CUs idle
+// or gives some one block more: us per RK4 step (thread-per-node kernel > this one, 4 / 5 fields)
+// are, at order 5, 81 > 85 / 85 > 101 for 1,296 elements, 103 > 88 / 111 > 108 for 2,058 and
+// 711 > 366 / 775 > 479 for 24,576; at order 4, 89 > 92 / 100 > 118 for 4,374, 113 > 99 /
+// 127 > 125 for 6,000 and 815 > 482 / 942 > 659 for 63,888. At order 3 (rows 20 of 32) it broke
+// even, at order 2 it was slower: not built. DGFEM_F64_MM=1 takes it at any size, =0 never.
+constexpr int64_t kF64MinElements4 = 6000, kF64MinElements5 = 2048;
+
+void pickF64(dg_context* c, const dg::RefElement& R) {
+    const char* kernel = std::getenv("DGFEM_KERNEL");
+    const char* env = std::getenv("DGFEM_F64_MM");
+    if (c->precision != DG_FP64 || c->dim != 3 || (kernel && kernel[0]) || (env && env[0] == '0')) return;
+    if (!(env && env[0] == '1') && c->K < (c->p == 5 ? kF64MinElements5 : kF64MinElements4)) return;
+    std::vector<double> frag;
+    if (!dgk::buildF64Frag(c->p, c->nf, R.Dw.data(), R.LIFT.data(), frag)) return;
+    c->f64Frag = uploadVec(c, frag);
+    c->f64Grid = (c->K + dgk::kF64Group - 1) / dgk::kF64Group;
+}
+
 // Grids that run in the resident time loop (dg_resident.hpp): at most as many 256-thread blocks as
 // the chip holds at once, without an explicit DGFEM_KERNEL or DGFEM_POST_BRANCH (both ask for
 // launches per stage). DGFEM_RESIDENT=0 switches it off.
@@ -1215,7 +1243,7 @@ void destroyContext(dg_context* c) {
     releaseGraphs(c);
     freeTables(c);
     for (void* p : {c->u, c->ulo, c->qa, c->snap, c->geo, c->fgeo, c->ops, c->afrag, c->afragBf,
-                    c->quadFrag, static_cast<void*>(c->fgeoH)})  // qa: with acc, qb
+                    c->quadFrag, static_cast<void*>(c->fgeoH), static_cast<void*>(c->f64Frag)})  // qa: with acc, qb
         devFree(p);
     devFree(c->nbr);
     devFree(c->iops);
@@ -1402,7 +1430,9 @@ dg_status dg_create(const dg_mesh_desc* m, const dg_physics* ph, const dg_option
             HIPCHK(hipMemset(c->dClosureW, 0, dgc::kNetWords * sizeof(dgk::u32x4_t)));
         }
         pickQuad(c, R);
-        c->nPartials = c->quadFrag ? std::max(c->quadGrid[dgk::kModeFinal], c->quadGrid[dgk::kModeEuler]) : c->nblocks;
+        pickF64(c, R);
+        c->nPartials = c->f64Frag ? c->f64Grid
+                       : c->quadFrag ? std::max(c->quadGrid[dgk::kModeFinal], c->quadGrid[dgk::kModeEuler]) : c->nblocks;
         c->resPartial = devAlloc<double>(c, static_cast<size_t>(c->nPartials) * 5);
         HIPCHK(hipMemset(c->resPartial, 0, static_cast<size_t>(c->nPartials) * 5 * sizeof(double)));
         if (c->nPartials > 4 * dgk::kResGroup) {  // below that the extra launch costs what it saves
