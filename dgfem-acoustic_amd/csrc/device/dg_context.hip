@@ -23,7 +23,7 @@
 #include "dg_kernels.hpp"
 #include "dg_kernels_bf16.hpp"
 #include "dg_resident.hpp"
-#include "dg_stage_f64.hpp"
+#include "dg_stage_tetmm.hpp"
 #include "dg_stage_quad.hpp"
 
 namespace {
@@ -108,8 +108,8 @@ struct dg_context {
     int64_t nPartials = 0;       // residual partials per step: blocks of the stage launch
     float* fgeoH = nullptr;      // (mixed; quad and resident kernels) per face h n, h (v0.n), h = Fscale / 2
     void* quadFrag = nullptr;    // operator of the lane-per-field stage kernel, or null: not used
-    double* f64Frag = nullptr;   // operator of the FP64 matrix-core stage kernel, or null: not used
-    int64_t f64Grid = 0;         // its blocks
+    void* tetFrag = nullptr;     // operator of the tetrahedra matrix-core stage kernel, or null: not used
+    int64_t tetGrid = 0;         // its blocks
     int64_t quadGrid[5] = {0, 0, 0, 0, 0};  // its blocks per mode (kMode*)
     // sources / observers (host definitions + device tables)
     std::vector<std::vector<int64_t>> srcNodes;
@@ -723,11 +723,13 @@ void runStage(dg_context* c, int stage, const void* qin, void* qout, void* uout,
         const int mode = dgk::stageMode(stage);
         dgk::launchStageQuad(mode, a, (c->K + dgk::kQuadGroup - 1) / dgk::kQuadGroup,
                              static_cast<unsigned>(c->quadGrid[mode]), c->stream);
-    } else if (c->f64Frag) {
-        dgk::StageArgs<double> a = stageArgs<double, false>(c, stage, qin, qout, uout, snap);
-        a.vfrag = c->f64Frag;
-        dgk::launchStageF64(c->p, c->nf, dgk::stageMode(stage), a,
-                            static_cast<unsigned>(c->f64Grid), c->stream);
+    } else if (c->tetFrag) {
+        auto launch = [&](auto a) {
+            a.vfrag = static_cast<decltype(a.vfrag)>(c->tetFrag);
+            dgk::launchStageTetMM(c->p, c->nf, dgk::stageMode(stage), a, static_cast<unsigned>(c->tetGrid), c->stream);
+        };
+        if (c->precision == DG_FP64) launch(stageArgs<double, false>(c, stage, qin, qout, uout, snap));
+        else launch(stageArgs<float, true>(c, stage, qin, qout, uout, snap));
     } else {
         c->stageFn(c, stage, qin, qout, uout, snap);
     }
@@ -1047,24 +1049,31 @@ void pickQuad(dg_context* c, const dg::RefElement& R) {
                                               static_cast<int64_t>(cus) * dgk::quadBlocksPerCu(mode));
 }
 
-// Grids that take the FP64 matrix-core stage kernel (dg_kernels_f64.hpp): tetrahedra of order 4 and
-// 5, without an explicit DGFEM_KERNEL. Its blocks take 16 elements, so a small grid leaves CUs idle
-// or gives some one block more: us per RK4 step (thread-per-node kernel > this one, 4 / 5 fields)
-// are, at order 5, 81 > 85 / 85 > 101 for 1,296 elements, 103 > 88 / 111 > 108 for 2,058 and
-// 711 > 366 / 775 > 479 for 24,576; at order 4, 89 > 92 / 100 > 118 for 4,374, 113 > 99 /
-// 127 > 125 for 6,000 and 815 > 482 / 942 > 659 for 63,888. At order 3 (rows 20 of 32) it broke
-// even, at order 2 it was slower: not built. DGFEM_F64_MM=1 takes it at any size, =0 never.
-constexpr int64_t kF64MinElements4 = 6000, kF64MinElements5 = 2048;
+// Grids that take the tetrahedra matrix-core stage kernel (dg_kernels_tetmm.hpp): order 4 and 5,
+// without an explicit DGFEM_KERNEL. Its blocks take 16 elements, so a small grid leaves CUs idle or
+// gives some one block more. us per RK4 step, kernel otherwise taken > this one, 4 / 5 fields:
+//   FP64  order 5: 1,296 elements 81 > 85 / 85 > 101; 2,058 103 > 83 / 111 > 104; 24,576 713 > 351 / 773 > 464
+//         order 4: 4,374 89 > 89 / 101 > 114; 6,000 113 > 99 / 127 > 125; 63,888 813 > 463 / 937 > 636
+//   mixed order 4: 4,374 56 > 59 / 64 > 70; 10,368 91 > 81 / 106 > 99; 162,000 862 > 636 / 1080 > 865
+// Not built: order 3 (20 of 32 rows used: broke even in FP64), order 2 (slower), and order 5 in mixed
+// precision, where it is faster than the split-BF16 kernel (48,000 elements 508 > 459) but its error
+// against FP64 larger (5 fields, 150 steps: 4.0e-7 against 2.5e-7; order 4, against the thread-per-node
+// kernel: 2.60e-7 and 2.65e-7). DGFEM_TET_MM=1 takes it at any size, =0 never.
+int64_t tetMMFrom(const dg_context* c) {
+    return c->precision == DG_MIXED ? 10000 : c->p == 5 ? 2048 : 6000;
+}
 
-void pickF64(dg_context* c, const dg::RefElement& R) {
+void pickTetMM(dg_context* c, const dg::RefElement& R) {
     const char* kernel = std::getenv("DGFEM_KERNEL");
-    const char* env = std::getenv("DGFEM_F64_MM");
-    if (c->precision != DG_FP64 || c->dim != 3 || (kernel && kernel[0]) || (env && env[0] == '0')) return;
-    if (!(env && env[0] == '1') && c->K < (c->p == 5 ? kF64MinElements5 : kF64MinElements4)) return;
-    std::vector<double> frag;
-    if (!dgk::buildF64Frag(c->p, c->nf, R.Dw.data(), R.LIFT.data(), frag)) return;
-    c->f64Frag = uploadVec(c, frag);
-    c->f64Grid = (c->K + dgk::kF64Group - 1) / dgk::kF64Group;
+    const char* env = std::getenv("DGFEM_TET_MM");
+    if (c->dim != 3 || (kernel && kernel[0]) || (env && env[0] == '0')) return;
+    if (!(env && env[0] == '1') && c->K < tetMMFrom(c)) return;
+    auto build = [&](auto frag) {
+        if (dgk::buildTetMMFrag(c->p, c->nf, R.Dw.data(), R.LIFT.data(), frag)) c->tetFrag = uploadVec(c, frag);
+    };
+    if (c->precision == DG_FP64) build(std::vector<double>());
+    else build(std::vector<float>());
+    c->tetGrid = (c->K + dgk::kTetMMGroup - 1) / dgk::kTetMMGroup;
 }
 
 // Grids that run in the resident time loop (dg_resident.hpp): at most as many 256-thread blocks as
@@ -1243,7 +1252,7 @@ void destroyContext(dg_context* c) {
     releaseGraphs(c);
     freeTables(c);
     for (void* p : {c->u, c->ulo, c->qa, c->snap, c->geo, c->fgeo, c->ops, c->afrag, c->afragBf,
-                    c->quadFrag, static_cast<void*>(c->fgeoH), static_cast<void*>(c->f64Frag)})  // qa: with acc, qb
+                    c->quadFrag, static_cast<void*>(c->fgeoH), c->tetFrag})  // qa: with acc, qb
         devFree(p);
     devFree(c->nbr);
     devFree(c->iops);
@@ -1430,8 +1439,8 @@ dg_status dg_create(const dg_mesh_desc* m, const dg_physics* ph, const dg_option
             HIPCHK(hipMemset(c->dClosureW, 0, dgc::kNetWords * sizeof(dgk::u32x4_t)));
         }
         pickQuad(c, R);
-        pickF64(c, R);
-        c->nPartials = c->f64Frag ? c->f64Grid
+        pickTetMM(c, R);
+        c->nPartials = c->tetFrag ? c->tetGrid
                        : c->quadFrag ? std::max(c->quadGrid[dgk::kModeFinal], c->quadGrid[dgk::kModeEuler]) : c->nblocks;
         c->resPartial = devAlloc<double>(c, static_cast<size_t>(c->nPartials) * 5);
         HIPCHK(hipMemset(c->resPartial, 0, static_cast<size_t>(c->nPartials) * 5 * sizeof(double)));
