@@ -368,6 +368,7 @@ struct ClosureArgs {
     const int32_t* __restrict__ iops;   // fmask
     const int64_t* __restrict__ faces;  // element * NFC + local face
     const dgk::u32x4_t* __restrict__ w; // network (packClosure)
+    const uint16_t* __restrict__ params;  // (closureWaveKernel) its BF16 parameters
     int64_t nfaces;
     dgk::Physics<T> ph;
 };
@@ -391,6 +392,235 @@ __global__ __launch_bounds__(kClosureBlock) void closureKernel(ClosureArgs<T> a)
     dgk::loadNode<NF>(a.qin + (e * NP + nd) * NF, qm);
     closureExterior<DIM, NFP, NF>(w, lds, a.ph, n, qm, qp);
     if (node < NFP && idx < a.nfaces) dgk::storeNode<NF>(a.ghost + (idx * NFP + node) * NF, qp);
+}
+
+// ---- FP64 contexts: the network's sums in one FP32 FMA chain per unit ----
+//
+// The FP32 rounding of these sums is the largest error of an FP64 run with learned faces (1e-9 of
+// the state), so any other order of summation, closureKernel's too (its error is half
+// as large), moves such a run's results by as much. FP64 contexts keep the chain and its results.
+//
+// FW faces per wave (4 or 8), kWaveWaves waves per block: the network is staged in LDS once per
+// block and every weight read serves a wave's faces together. With few faces (a 2D truncation
+// boundary) 4 faces per wave spread the work over twice the waves.
+constexpr int kWaveWaves = 4;
+constexpr int kWaveBlock = 64 * kWaveWaves;
+constexpr int kWaveSmall = 4096;  // at most this many faces: 4 faces per wave, else 8
+
+// Forward pass of F samples by one wave (lane = hidden unit): each weight read from LDS serves
+// F samples and the F accumulations are independent. Inputs sx[F][XS] (XS >= NIN, a multiple of
+// 4), activations sa[F][kH], outputs sy[F][NOUT]; sx and sa2 may share storage (sx is consumed
+// before sa2 is written). Per output the sum runs over the inputs in ascending order, as in
+// mlpForwardWave.
+template <int NIN, int NOUT, int F, int XS>
+__device__ inline void mlpForwardBatch(const float* net, const float* sx, float* sa1, float* sa2, float* sy, int lane) {
+    using N = NetLds<NIN, NOUT>;
+    static_assert(XS % 4 == 0 && XS >= NIN && NOUT <= 16 && F % 4 == 0, "batch layout");
+    typedef float F4 __attribute__((ext_vector_type(4)));
+    float z[F];
+    {
+        const float* w = net + N::kW1 + lane * N::S1;
+        const float b = net[N::kB1 + lane];
+#pragma unroll
+        for (int f = 0; f < F; ++f) z[f] = b;
+        constexpr int NIN4 = NIN & ~3;
+#pragma unroll 2
+        for (int i = 0; i < NIN4; i += 4) {
+            const float w0 = w[i], w1 = w[i + 1], w2 = w[i + 2], w3 = w[i + 3];
+#pragma unroll
+            for (int f = 0; f < F; ++f) {
+                const F4 x = *reinterpret_cast<const F4*>(sx + f * XS + i);
+                z[f] = fmaf(w3, x[3], fmaf(w2, x[2], fmaf(w1, x[1], fmaf(w0, x[0], z[f]))));
+            }
+        }
+#pragma unroll
+        for (int i = NIN4; i < NIN; ++i) {
+            const float wi = w[i];
+#pragma unroll
+            for (int f = 0; f < F; ++f) z[f] = fmaf(wi, sx[f * XS + i], z[f]);
+        }
+#pragma unroll
+        for (int f = 0; f < F; ++f) sa1[f * kH + lane] = tanhf(z[f]);
+    }
+    waveFence();
+    {
+        const float* w = net + N::kW2 + lane * N::S2;
+        const float b = net[N::kB2 + lane];
+#pragma unroll
+        for (int f = 0; f < F; ++f) z[f] = b;
+#pragma unroll 2
+        for (int k = 0; k < kH; k += 4) {
+            const float w0 = w[k], w1 = w[k + 1], w2 = w[k + 2], w3 = w[k + 3];
+#pragma unroll
+            for (int f = 0; f < F; ++f) {
+                const F4 x = *reinterpret_cast<const F4*>(sa1 + f * kH + k);
+                z[f] = fmaf(w3, x[3], fmaf(w2, x[2], fmaf(w1, x[1], fmaf(w0, x[0], z[f]))));
+            }
+        }
+#pragma unroll
+        for (int f = 0; f < F; ++f) sa2[f * kH + lane] = tanhf(z[f]);
+    }
+    waveFence();
+    {
+        // lane = output j + 16 g: samples g, g + 4, ...
+        const int j = lane & 15, g = lane >> 4;
+        if (j < NOUT) {
+            constexpr int FG = F / 4;
+            const float* w = net + N::kW3 + j * N::S2;
+            const float b = net[N::kB3 + j];
+            float y[FG];
+#pragma unroll
+            for (int c = 0; c < FG; ++c) y[c] = b;
+#pragma unroll 2
+            for (int k = 0; k < kH; k += 4) {
+                const float w0 = w[k], w1 = w[k + 1], w2 = w[k + 2], w3 = w[k + 3];
+#pragma unroll
+                for (int c = 0; c < FG; ++c) {
+                    const F4 x = *reinterpret_cast<const F4*>(sa2 + (g + 4 * c) * kH + k);
+                    y[c] = fmaf(w3, x[3], fmaf(w2, x[2], fmaf(w1, x[1], fmaf(w0, x[0], y[c]))));
+                }
+            }
+#pragma unroll
+            for (int c = 0; c < FG; ++c) sy[(g + 4 * c) * NOUT + j] = y[c];
+        }
+    }
+    waveFence();
+}
+
+// Exterior states of the learned faces for one stage. Face-node work runs with lane =
+// (face slot, node): 16 lanes per face (NFP <= 16), 4 faces per pass.
+template <int DIM, int P, int NF, typename T, int FW>
+__global__ __launch_bounds__(kWaveBlock) void closureWaveKernel(ClosureArgs<T> a) {
+    using S = dgk::Sizes<DIM, P>;
+    using L = dgk::OpLayout<DIM, P>;
+    constexpr int NP = S::NP, NFP = S::NFP, NFC = S::NFC;
+    constexpr int NT = DIM - 1;  // tangential directions
+    constexpr int NIN = DIM * NFP + 2, NOUT = NFP;
+    constexpr int NPASS = FW / 4;
+    static_assert(FW % 4 == 0, "4 faces per pass");
+    constexpr int XS = (NIN + 3) & ~3;
+    static_assert(NFP <= 16 && XS <= kH, "closure lane layout");
+    using N = NetLds<NIN, NOUT>;
+    __shared__ float net[N::kTotal];
+    __shared__ __align__(16) float bufX[kWaveWaves][FW * kH];   // inputs, then second activations
+    __shared__ __align__(16) float bufA[kWaveWaves][FW * kH];   // first activations
+    __shared__ float bufY[kWaveWaves][FW * NOUT];
+    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+    const int slot = lane >> 4, node = lane & 15;
+    const bool nodeLane = node < NFP;
+    const int64_t f0 = static_cast<int64_t>(blockIdx.x) * (kWaveWaves * FW) + wave * FW;
+    // face records of this lane's faces, issued with the network loads
+    int64_t ef[NPASS];
+#pragma unroll
+    for (int ps = 0; ps < NPASS; ++ps) {
+        const int64_t idx = f0 + ps * 4 + slot;
+        ef[ps] = a.faces[idx < a.nfaces ? idx : a.nfaces - 1];
+    }
+    loadNet<NIN, NOUT, kWaveBlock>(a.params, net, tid);
+    __syncthreads();
+    float* sx = bufX[wave];
+    const T c0 = a.ph.c0;
+    // per pass: this lane's face frame and node characteristics
+    T n[NPASS][3], t[NPASS][NT][3], vn0[NPASS], wo[NPASS], wi[NPASS], tt[NPASS][NT], qm[NPASS][NF];
+    float sc[NPASS];
+#pragma unroll
+    for (int ps = 0; ps < NPASS; ++ps) {
+        const int64_t e = ef[ps] / NFC;
+        const int f = static_cast<int>(ef[ps] - e * NFC);
+        n[ps][0] = a.fgeo[(e * NFC + f) * 4];
+        n[ps][1] = a.fgeo[(e * NFC + f) * 4 + 1];
+        n[ps][2] = DIM == 3 ? a.fgeo[(e * NFC + f) * 4 + 2] : T(0);
+        const int nd = a.iops[L::kMask + f * NFP + (nodeLane ? node : 0)];
+        const T* q = a.qin + (e * NP + nd) * NF;
+#pragma unroll
+        for (int k = 0; k < NF; ++k) qm[ps][k] = q[k];
+    }
+#pragma unroll
+    for (int ps = 0; ps < NPASS; ++ps) {
+        T vt0;
+        if constexpr (DIM == 2) {
+            t[ps][0][0] = -n[ps][1];
+            t[ps][0][1] = n[ps][0];
+            t[ps][0][2] = T(0);
+            vn0[ps] = a.ph.v0[0] * n[ps][0] + a.ph.v0[1] * n[ps][1];
+            vt0 = a.ph.v0[0] * t[ps][0][0] + a.ph.v0[1] * t[ps][0][1];
+        } else {
+            vn0[ps] = a.ph.v0[0] * n[ps][0] + a.ph.v0[1] * n[ps][1] + a.ph.v0[2] * n[ps][2];
+            // t1 along the tangential mean flow, else along the axis least aligned with n
+            T u[3];
+            for (int c = 0; c < 3; ++c) u[c] = a.ph.v0[c] - vn0[ps] * n[ps][c];
+            vt0 = sqrt(u[0] * u[0] + u[1] * u[1] + u[2] * u[2]);
+            if (!(vt0 > T(1e-6) * c0)) {
+                const T ax = fabs(n[ps][0]), ay = fabs(n[ps][1]), az = fabs(n[ps][2]);
+                const int k = (ax <= ay && ax <= az) ? 0 : (ay <= az ? 1 : 2);
+                for (int c = 0; c < 3; ++c) u[c] = (c == k ? T(1) : T(0)) - n[ps][k] * n[ps][c];
+                vt0 = T(0);
+            }
+            const T iu = T(1) / sqrt(u[0] * u[0] + u[1] * u[1] + u[2] * u[2]);
+            for (int c = 0; c < 3; ++c) t[ps][0][c] = u[c] * iu;
+            t[ps][1][0] = n[ps][1] * t[ps][0][2] - n[ps][2] * t[ps][0][1];
+            t[ps][1][1] = n[ps][2] * t[ps][0][0] - n[ps][0] * t[ps][0][2];
+            t[ps][1][2] = n[ps][0] * t[ps][0][1] - n[ps][1] * t[ps][0][0];
+        }
+        const T Pv = qm[ps][0] * a.ph.irc0;
+        T Nn = qm[ps][1] * n[ps][0] + qm[ps][2] * n[ps][1];
+        if constexpr (DIM == 3) Nn += qm[ps][3] * n[ps][2];
+        wo[ps] = nodeLane ? Pv + Nn : T(0);
+        wi[ps] = Pv - Nn;
+        for (int c = 0; c < NT; ++c) {
+            T v = qm[ps][1] * t[ps][c][0] + qm[ps][2] * t[ps][c][1];
+            if constexpr (DIM == 3) v += qm[ps][3] * t[ps][c][2];
+            tt[ps][c] = nodeLane ? v : T(0);
+        }
+        // scale: RMS over the face's nodes of the outgoing and tangential characteristics
+        const float wof = static_cast<float>(wo[ps]);
+        float ss = wof * wof;
+        for (int c = 0; c < NT; ++c) {
+            const float ttf = static_cast<float>(tt[ps][c]);
+            ss += ttf * ttf;
+        }
+#pragma unroll
+        for (int off = 8; off > 0; off >>= 1) ss += __shfl_xor(ss, off, 64);
+        sc[ps] = sqrtf(ss / NFP) + 1e-30f;
+        const float is = 1.0f / sc[ps];
+        float* x = sx + (ps * 4 + slot) * XS;
+        if (nodeLane) {
+            x[node] = wof * is;
+            for (int c = 0; c < NT; ++c) x[(1 + c) * NFP + node] = static_cast<float>(tt[ps][c]) * is;
+        } else if (node == NFP) {
+            const float ic0 = static_cast<float>(T(1) / c0);
+            x[DIM * NFP] = static_cast<float>(vn0[ps]) * ic0;
+            x[DIM * NFP + 1] = static_cast<float>(vt0) * ic0;
+        } else if (node == NFP + 1) {
+            for (int i = NIN; i < XS; ++i) x[i] = 0.0f;
+        }
+    }
+    waveFence();
+    mlpForwardBatch<NIN, NOUT, FW, XS>(net, sx, bufA[wave], sx, bufY[wave], lane);
+#pragma unroll
+    for (int ps = 0; ps < NPASS; ++ps) {
+        const int64_t idx = f0 + ps * 4 + slot;
+        if (!nodeLane || idx >= a.nfaces) continue;
+        const T what = static_cast<T>(sc[ps] * bufY[wave][(ps * 4 + slot) * NOUT + node]);
+        const T lam = vn0[ps] - c0;
+        const T wip = (T(2) * lam * what - (lam + c0) * wi[ps]) / (lam - c0);
+        T tp[NT];
+        for (int c = 0; c < NT; ++c)
+            tp[c] = (vn0[ps] >= T(0)) ? tt[ps][c] : -(vn0[ps] + c0) * tt[ps][c] / (vn0[ps] - c0);
+        const T Pp = T(0.5) * (wo[ps] + wip), Np_ = T(0.5) * (wo[ps] - wip);
+        T qp[NF];
+        qp[0] = a.ph.rho0 * c0 * Pp;
+        for (int x = 0; x < DIM; ++x) {
+            T v = Np_ * n[ps][x];
+            for (int c = 0; c < NT; ++c) v += tp[c] * t[ps][c][x];
+            qp[1 + x] = v;
+        }
+        if constexpr (DIM == 2) qp[3] = qm[ps][3];
+        if constexpr (NF == 5) qp[4] = qm[ps][4] + (qp[0] - qm[ps][0]) * a.ph.ic2;
+        T* g = a.ghost + (idx * NFP + node) * NF;
+#pragma unroll
+        for (int k = 0; k < NF; ++k) g[k] = qp[k];
+    }
 }
 
 // Interior and exterior traces (exterior in the interior element's face-node order) and

@@ -170,7 +170,8 @@ struct dg_context {
     int64_t nLearned = 0;
     int64_t* dLearned = nullptr;
     void* ghost = nullptr;
-    dgk::u32x4_t* dClosureW = nullptr;  // the network's matrix-core operands (packClosure)
+    dgk::u32x4_t* dClosureW = nullptr;  // (mixed) the network's matrix-core operands (packClosure)
+    uint16_t* dClosureParams = nullptr;  // (FP64) its BF16 parameters
     int64_t closureParams = 0;
     ClosureFn closureFn = nullptr;
     TraceFn traceFn = nullptr;
@@ -530,9 +531,20 @@ void launchClosure(dg_context* c, const void* qin) {
     a.w = c->dClosureW;
     a.nfaces = c->nLearned;
     a.ph = makePhysics<T>(c->phys);
-    const int64_t nb = (c->nLearned + dgc::kTileFaces - 1) / dgc::kTileFaces;
-    hipLaunchKernelGGL((dgc::closureKernel<DIM, P, NF, T>), dim3(static_cast<unsigned>(nb)), dim3(dgc::kClosureBlock), 0,
-                       c->stream, a);
+    if constexpr (std::is_same_v<T, double>) {
+        a.params = c->dClosureParams;
+        auto launch = [&](auto kernel, int faces) {
+            const int64_t perBlock = static_cast<int64_t>(dgc::kWaveWaves) * faces;
+            hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>((c->nLearned + perBlock - 1) / perBlock)),
+                               dim3(dgc::kWaveBlock), 0, c->stream, a);
+        };
+        if (c->nLearned <= dgc::kWaveSmall) launch(dgc::closureWaveKernel<DIM, P, NF, T, 4>, 4);
+        else launch(dgc::closureWaveKernel<DIM, P, NF, T, 8>, 8);
+    } else {
+        const int64_t nb = (c->nLearned + dgc::kTileFaces - 1) / dgc::kTileFaces;
+        hipLaunchKernelGGL((dgc::closureKernel<DIM, P, NF, T>), dim3(static_cast<unsigned>(nb)),
+                           dim3(dgc::kClosureBlock), 0, c->stream, a);
+    }
 }
 
 template <int DIM, int P, int NF, typename T>
@@ -1087,6 +1099,7 @@ void pickResident(dg_context* c) {
         if (v && v[0]) return;
     }
     if (c->kernelKind != DG_KERNEL_VALU && c->kernelKind != DG_KERNEL_VM) return;
+    if (c->precision == DG_FP64 && c->nLearned > 0) return;  // (closureWaveKernel: a launch of its own)
     int cus = 0, coop = 0;
     HIPCHK(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, c->device));
     HIPCHK(hipDeviceGetAttribute(&coop, hipDeviceAttributeCooperativeLaunch, c->device));
@@ -1271,6 +1284,7 @@ void destroyContext(dg_context* c) {
     devFree(c->dLearned);
     devFree(c->ghost);
     devFree(c->dClosureW);
+    devFree(c->dClosureParams);
     devFree(c->resMail);
     devFree(c->dSrcVal);
     for (void* h : {static_cast<void*>(c->hT), static_cast<void*>(c->hV), static_cast<void*>(c->hRes),
@@ -1435,8 +1449,13 @@ dg_status dg_create(const dg_mesh_desc* m, const dg_physics* ph, const dg_option
             c->dLearned = uploadVec(c, c->mesh.learnedFaces);
             c->ghost = alloc(static_cast<size_t>(c->nLearned) * c->Nfp * c->nf);
             c->closureParams = dgc::numParams(c->dim * c->Nfp + 2, c->Nfp);
-            c->dClosureW = devAlloc<dgk::u32x4_t>(c, dgc::kNetWords);
-            HIPCHK(hipMemset(c->dClosureW, 0, dgc::kNetWords * sizeof(dgk::u32x4_t)));
+            if (c->precision == DG_FP64) {
+                c->dClosureParams = devAlloc<uint16_t>(c, c->closureParams);
+                HIPCHK(hipMemset(c->dClosureParams, 0, c->closureParams * sizeof(uint16_t)));
+            } else {
+                c->dClosureW = devAlloc<dgk::u32x4_t>(c, dgc::kNetWords);
+                HIPCHK(hipMemset(c->dClosureW, 0, dgc::kNetWords * sizeof(dgk::u32x4_t)));
+            }
         }
         pickQuad(c, R);
         pickTetMM(c, R);
@@ -1496,9 +1515,13 @@ dg_status dg_set_closure(dg_context* c, const uint16_t* params, int64_t n) {
     try {
         HIPCHK(hipSetDevice(c->device));
         HIPCHK(hipStreamSynchronize(c->stream));
-        std::vector<uint32_t> words(dgc::kNetWords * 4, 0);
-        dgc::packClosure(c->dim * c->Nfp + 2, c->Nfp, params, words.data());
-        HIPCHK(hipMemcpy(c->dClosureW, words.data(), words.size() * sizeof(uint32_t), hipMemcpyHostToDevice));
+        if (c->precision == DG_FP64) {
+            HIPCHK(hipMemcpy(c->dClosureParams, params, n * sizeof(uint16_t), hipMemcpyHostToDevice));
+        } else {
+            std::vector<uint32_t> words(dgc::kNetWords * 4, 0);
+            dgc::packClosure(c->dim * c->Nfp + 2, c->Nfp, params, words.data());
+            HIPCHK(hipMemcpy(c->dClosureW, words.data(), words.size() * sizeof(uint32_t), hipMemcpyHostToDevice));
+        }
     } catch (const std::exception& ex) {
         return fail(c, DG_ERR_DEVICE, ex.what());
     }

@@ -16,7 +16,7 @@
 // of the same face node; the owner writes the same mailbox two epochs later, after it received
 // that trace, so a mailbox is always empty when it is written.
 //
-// Learned faces (DG_BC_LEARNED): further blocks of the launch evaluate the closure network for 16
+// Learned faces (DG_BC_LEARNED, mixed precision): further blocks of the launch evaluate the closure network for 16
 // faces each. To the block that owns such a face they are one more neighbour: they receive its trace
 // in an inbox and answer into the mailboxes of its face nodes. (Evaluated by the owning block itself
 // the network's registers came on top of the block's state: its spills made 1,000-block grids slower
@@ -249,7 +249,7 @@ __global__ __launch_bounds__(kBlock, (ResidentShape<DIM, P, NF, T, SHAPE>::kWave
 
     if (static_cast<int>(blockIdx.x) >= a.blocks) {
         // ---- a block of learned faces: trace in, exterior state out, once per stage ----
-        if constexpr (DIM == 2 || P <= 3) {
+        if constexpr (sizeof(T) == 4) {  // (FP64 grids with learned faces launch per stage: closureWaveKernel)
             dgc::ClosureLds& lds = *reinterpret_cast<dgc::ClosureLds*>(sQF);
             const int node = tid & 15, idx = (static_cast<int>(blockIdx.x) - a.blocks) * dgc::kTileFaces + (tid >> 4);
             const bool mine = idx < a.nLearned && node < NFP;
