@@ -208,7 +208,9 @@ def main():
 
     mixed = out["mixed"]
     kernel_name = {"valu": "stageKernel<3,3,4,float,true>",
-                   "vm": "stageKernel<3,3,4,float,true,VM>",
+                   # dg_get_info names the variant of the order; large grids run the lane-per-field kernel
+                   "vm": "stageKernelQuad<3,3>" if m.K >= 163840 and not os.environ.get("DGFEM_KERNEL")
+                         and os.environ.get("DGFEM_QUAD") != "0" else "stageKernel<3,3,4,float,true,VM>",
                    "wave": "stageKernelWave<3,3,float,true>",
                    "mm": "stageKernelMM<3,3,float,true>",
                    "bf16x6": "stageKernelBf16<3,3,4,3>",

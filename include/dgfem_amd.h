@@ -49,7 +49,12 @@ enum { DG_RK4 = 0, DG_EULER = 1 };                  /* config timeIntMethod */
    three products). Environment DGFEM_KERNEL = valu | vm | mm | wave | bf16x6 | bf16x3; an explicit
    request that is not built for the mesh or precision fails dg_create with DG_ERR_UNSUPPORTED.
    Without it: bf16x6 for the mixed precision on tetrahedra of order 5, vm on tetrahedra of
-   order 3, valu otherwise. */
+   order 3, valu otherwise; and, by size and order, three forms that have no name here and are not
+   used with DGFEM_KERNEL: a stage kernel with a lane per (element, field) (mixed precision, 4
+   fields, from 163,840 tetrahedra of order 3; DGFEM_QUAD = 0 | 1), a stage kernel with both
+   contractions on the FP64 / FP32 matrix cores (from 2,048 tetrahedra of order 5 and 6,000 of
+   order 4 in FP64, 10,000 of order 4 in mixed precision; DGFEM_TET_MM = 0 | 1), and one resident
+   launch for many steps on grids that the chip holds at once (DGFEM_RESIDENT = 0: off). */
 enum { DG_KERNEL_VALU = 0, DG_KERNEL_MM = 1, DG_KERNEL_WAVE = 2, DG_KERNEL_BF16X6 = 3, DG_KERNEL_BF16X3 = 4,
        DG_KERNEL_VM = 5 };
 
@@ -154,7 +159,9 @@ typedef struct {
     int64_t num_elements, num_faces, num_boundary_faces;
     double min_inradius;
     int64_t device_bytes;
-    int32_t stage_kernel;        /* DG_KERNEL_* chosen by dg_create */
+    int32_t stage_kernel;        /* DG_KERNEL_* chosen by dg_create; this and the two numbers of
+                                    blocks below describe that variant, also where one of the forms
+                                    without a name runs the steps in its place */
     int32_t post_branch;         /* 1: captured RK4 steps run the end-of-step kernel on a graph branch
                                     of its own (stage grids of >= 4096 blocks, no observer node that
                                     is also a source node, graphs on) */
