@@ -103,9 +103,9 @@ struct dg_context {
     int32_t *nbr = nullptr, *iops = nullptr;
     uint8_t *code = nullptr, *toCanon = nullptr;
     double* resPartial = nullptr;
-    double* resGroup = nullptr;  // per-group residual sums when nPartials > 4 kResGroup
-    int64_t nblocks = 0, nResGroups = 0;
-    int64_t nPartials = 0;       // residual partials per step: blocks of the stage launch
+    double* resGroup = nullptr;  // per-group residual sums when a step has more than 4 kResGroup partials
+    int64_t nblocks = 0;
+    int64_t nPartials = 0;       // residual partials of a step: blocks of the last final-stage launch
     float* fgeoH = nullptr;      // (mixed; quad and resident kernels) per face h n, h (v0.n), h = Fscale / 2
     void* quadFrag = nullptr;    // operator of the lane-per-field stage kernel, or null: not used
     void* tetFrag = nullptr;     // operator of the tetrahedra matrix-core stage kernel, or null: not used
@@ -496,10 +496,11 @@ void launchPost(dg_context* c) {
     p.resPartial = c->resPartial;
     p.nblocks = c->nPartials;
     if (c->resGroup && c->curResid) {
-        hipLaunchKernelGGL(dgk::residualGroupKernel, dim3(static_cast<unsigned>(c->nResGroups)), dim3(256), 0, st,
+        const int64_t groups = (c->nPartials + dgk::kResGroup - 1) / dgk::kResGroup;
+        hipLaunchKernelGGL(dgk::residualGroupKernel, dim3(static_cast<unsigned>(groups)), dim3(256), 0, st,
                            static_cast<const double*>(c->resPartial), c->nPartials, c->resGroup);
         p.resPartial = c->resGroup;
-        p.nblocks = c->nResGroups;
+        p.nblocks = groups;
     }
     p.invN = 1.0 / static_cast<double>(c->K * c->Np);
     p.obsIdx = c->dObsIdx;
@@ -733,6 +734,8 @@ void runStage(dg_context* c, int stage, const void* qin, void* qout, void* uout,
         a.vfrag = static_cast<const float*>(c->quadFrag);
         a.fgeo = c->fgeoH;
         const int mode = dgk::stageMode(stage);
+        // (the persistent grids of the two final stages differ: only the rows of this one are a step's)
+        if (mode == dgk::kModeFinal || mode == dgk::kModeEuler) c->nPartials = c->quadGrid[mode];
         dgk::launchStageQuad(mode, a, (c->K + dgk::kQuadGroup - 1) / dgk::kQuadGroup,
                              static_cast<unsigned>(c->quadGrid[mode]), c->stream);
     } else if (c->tetFrag) {
@@ -1459,13 +1462,13 @@ dg_status dg_create(const dg_mesh_desc* m, const dg_physics* ph, const dg_option
         }
         pickQuad(c, R);
         pickTetMM(c, R);
+        // (the larger of a quad context's two until its first final stage)
         c->nPartials = c->tetFrag ? c->tetGrid
                        : c->quadFrag ? std::max(c->quadGrid[dgk::kModeFinal], c->quadGrid[dgk::kModeEuler]) : c->nblocks;
         c->resPartial = devAlloc<double>(c, static_cast<size_t>(c->nPartials) * 5);
         HIPCHK(hipMemset(c->resPartial, 0, static_cast<size_t>(c->nPartials) * 5 * sizeof(double)));
         if (c->nPartials > 4 * dgk::kResGroup) {  // below that the extra launch costs what it saves
-            c->nResGroups = (c->nPartials + dgk::kResGroup - 1) / dgk::kResGroup;
-            c->resGroup = devAlloc<double>(c, static_cast<size_t>(c->nResGroups) * 5);
+            c->resGroup = devAlloc<double>(c, static_cast<size_t>((c->nPartials + dgk::kResGroup - 1) / dgk::kResGroup) * 5);
         }
         c->ringSlots = 4096;
         c->resRing = devAlloc<double>(c, c->ringSlots * 5);
