@@ -186,7 +186,8 @@ def main():
         s = make_solver(m, bc, prec, args.steps_per_graph)
         if want:
             os.environ.pop("DGFEM_KERNEL", None)
-        kernels[name] = dg.KERNEL_NAMES[s.info().stage_kernel]
+        quad = s.forms().stage_form == dg.DG_FORM_QUAD
+        kernels[name] = "quad" if quad else dg.KERNEL_NAMES[s.info().stage_kernel]
         states[name], r, wall = accuracy_then_timed_run(s, args.accuracy_steps, args.steps, args.warmup, dt)
         ms = s.profile_steps(dt, args.profile_steps)
         stage_ms = ms[0]
@@ -208,9 +209,8 @@ def main():
 
     mixed = out["mixed"]
     kernel_name = {"valu": "stageKernel<3,3,4,float,true>",
-                   # dg_get_info names the variant of the order; large grids run the lane-per-field kernel
-                   "vm": "stageKernelQuad<3,3>" if m.K >= 163840 and not os.environ.get("DGFEM_KERNEL")
-                         and os.environ.get("DGFEM_QUAD") != "0" else "stageKernel<3,3,4,float,true,VM>",
+                   "vm": "stageKernel<3,3,4,float,true,VM>",
+                   "quad": "stageKernelQuad<3,3>",
                    "wave": "stageKernelWave<3,3,float,true>",
                    "mm": "stageKernelMM<3,3,float,true>",
                    "bf16x6": "stageKernelBf16<3,3,4,3>",

@@ -139,6 +139,7 @@ struct dg_context {
     int64_t resBlocks = 0, resGrid = 0;  // blocks of elements; with those of learned faces
     int resShape = 0;                  // dgk::kRes*
     int resChunk = 0;                  // steps per launch
+    int64_t resLaunches = 0, resAborts = 0;  // launches that ran to their end; batches handed back
     unsigned char* resMail = nullptr;  // two sets of mailboxes, then outcomes and counts per chunk
     size_t resMailBytes = 0;           //   of one set
     int *resOutcome = nullptr, *resDone = nullptr;
@@ -1128,6 +1129,8 @@ void pickResident(dg_context* c) {
     c->resDone = c->resOutcome + chunks;
 }
 
+bool useResident(const dg_context* c) { return c->resBlocks > 0 && c->resChunk >= kResMinChunk; }
+
 template <typename T>
 hipError_t launchChunk(dg_context* c, int chunk, int64_t slot0, int steps, int64_t batch, int integrator, bool resid) {
     dgk::ResidentArgs<T> a{};
@@ -1731,7 +1734,7 @@ dg_status dg_run(dg_context* c, const dg_run_params* prm, dg_step_fn on_step, dg
         c->curResid = resid ? 1 : 0;
         c->curDt = prm->dt;
         const bool useGraph = c->opt.use_graph != 0;
-        const bool resident = c->resBlocks > 0 && c->resChunk >= kResMinChunk;
+        const bool resident = useResident(c);
         auto readyGraphs = [&] {
             if (useGraph && (c->gOne == nullptr || c->gIntegrator != prm->integrator || c->gResid != (resid ? 1 : 0) ||
                              c->gSteps != c->opt.steps_per_graph || c->gDt != prm->dt))
@@ -1801,7 +1804,9 @@ dg_status dg_run(dg_context* c, const dg_run_params* prm, dg_step_fn on_step, dg
                 HIPCHK(hipStreamSynchronize(c->stream));
                 const int64_t good = std::find_if(outcome.begin(), outcome.end(), [](int o) { return o != dgk::kDone; }) -
                                      outcome.begin();
+                c->resLaunches += good;
                 if (good < static_cast<int64_t>(outcome.size())) {
+                    ++c->resAborts;
                     // a block waited too long: the state is the one before chunk `good`
                     readyGraphs();
                     hipLaunchKernelGGL(dgk::setCounterKernel, dim3(1), dim3(1), 0, c->stream, c->counter, c->batchSteps, n,
@@ -1915,6 +1920,18 @@ dg_status dg_get_info(const dg_context* c, dg_info* info) {
     info->post_branch = (c->opt.use_graph != 0 && usePostBranch(c, DG_RK4)) ? 1 : 0;
     info->elements_per_block = c->eb;
     info->stage_blocks = c->nblocks;
+    return DG_OK;
+}
+
+dg_status dg_get_forms(const dg_context* c, dg_forms* forms) {
+    if (!c || !forms) return DG_ERR_INVALID;
+    forms->stage_form = c->quadFrag ? DG_FORM_QUAD : c->tetFrag ? DG_FORM_TET_MM : DG_FORM_KERNEL;
+    forms->resident = useResident(c) ? 1 : 0;
+    forms->resident_shape = c->resBlocks > 0 ? c->resShape : -1;
+    forms->stage_blocks = c->quadFrag ? c->quadGrid[dgk::kModeFinal] : c->tetFrag ? c->tetGrid : c->nblocks;
+    forms->resident_blocks = c->resBlocks > 0 ? c->resGrid : 0;
+    forms->resident_launches = c->resLaunches;
+    forms->resident_aborts = c->resAborts;
     return DG_OK;
 }
 

@@ -26,6 +26,7 @@ DG_RK4, DG_EULER = 0, 1
 DG_KERNEL_VALU, DG_KERNEL_MM, DG_KERNEL_WAVE, DG_KERNEL_BF16X6, DG_KERNEL_BF16X3, DG_KERNEL_VM = 0, 1, 2, 3, 4, 5
 KERNEL_NAMES = {DG_KERNEL_VALU: "valu", DG_KERNEL_MM: "mm", DG_KERNEL_WAVE: "wave", DG_KERNEL_BF16X6: "bf16x6",
                 DG_KERNEL_BF16X3: "bf16x3", DG_KERNEL_VM: "vm"}
+DG_FORM_KERNEL, DG_FORM_QUAD, DG_FORM_TET_MM = 0, 1, 2
 
 
 class DGError(RuntimeError):
@@ -72,6 +73,12 @@ class Info(C.Structure):
                 ("post_branch", C.c_int32), ("elements_per_block", C.c_int32), ("stage_blocks", C.c_int64)]
 
 
+class Forms(C.Structure):
+    _fields_ = [("stage_form", C.c_int32), ("resident", C.c_int32), ("resident_shape", C.c_int32),
+                ("stage_blocks", C.c_int64), ("resident_blocks", C.c_int64), ("resident_launches", C.c_int64),
+                ("resident_aborts", C.c_int64)]
+
+
 VALUE_FN = C.CFUNCTYPE(C.c_int, C.c_void_p, C.c_double, C.POINTER(C.c_double))
 STEP_FN = C.CFUNCTYPE(C.c_int, C.c_void_p, C.POINTER(StepRecord))
 SAVE_FN = C.CFUNCTYPE(C.c_int, C.c_void_p, C.c_int64, C.c_double, C.POINTER(C.c_double))
@@ -104,6 +111,7 @@ def load_library(path: str = LIB_PATH) -> C.CDLL:
                                        C.c_int64, P(C.c_int64)]),
         "dg_rhs": (C.c_int32, [C.c_void_p, P(C.c_double), P(C.c_double), C.c_double]),
         "dg_get_info": (C.c_int32, [C.c_void_p, P(Info)]),
+        "dg_get_forms": (C.c_int32, [C.c_void_p, P(Forms)]),
         "dg_profile_steps": (C.c_int32, [C.c_void_p, C.c_double, C.c_int32, P(C.c_double), P(C.c_double),
                                          P(C.c_double)]),
         "dg_last_run_device_ms": (C.c_double, [C.c_void_p]),
@@ -512,6 +520,12 @@ class Solver:
         inf = Info()
         self._check(self._lib.dg_get_info(self._h, C.byref(inf)))
         return inf
+
+    def forms(self) -> Forms:
+        """Which code runs the steps, and how often the resident loop ran or handed back."""
+        f = Forms()
+        self._check(self._lib.dg_get_forms(self._h, C.byref(f)))
+        return f
 
     def rhs(self, u, dt) -> np.ndarray:
         u = np.ascontiguousarray(u, dtype=np.float64).reshape(self.state_shape)

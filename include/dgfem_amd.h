@@ -49,8 +49,8 @@ enum { DG_RK4 = 0, DG_EULER = 1 };                  /* config timeIntMethod */
    three products). Environment DGFEM_KERNEL = valu | vm | mm | wave | bf16x6 | bf16x3; an explicit
    request that is not built for the mesh or precision fails dg_create with DG_ERR_UNSUPPORTED.
    Without it: bf16x6 for the mixed precision on tetrahedra of order 5, vm on tetrahedra of
-   order 3, valu otherwise; and, by size and order, three forms that have no name here and are not
-   used with DGFEM_KERNEL: a stage kernel with a lane per (element, field) (mixed precision, 4
+   order 3, valu otherwise; and, by size and order, three forms that have no name here, are not
+   used with DGFEM_KERNEL and are reported by dg_get_forms: a stage kernel with a lane per (element, field) (mixed precision, 4
    fields, from 163,840 tetrahedra of order 3; DGFEM_QUAD = 0 | 1), a stage kernel with both
    contractions on the FP64 / FP32 matrix cores (from 2,048 tetrahedra of order 5 and 6,000 of
    order 4 in FP64, 10,000 of order 4 in mixed precision; DGFEM_TET_MM = 0 | 1), and one resident
@@ -169,6 +169,24 @@ typedef struct {
     int64_t stage_blocks;        /* blocks per stage launch */
 } dg_info;
 DG_API dg_status dg_get_info(const dg_context* ctx, dg_info* info);
+
+/* Which code runs the context's steps. */
+enum { DG_FORM_KERNEL = 0,   /* the kernel dg_info.stage_kernel names */
+       DG_FORM_QUAD = 1,     /* stage kernel with a lane per (element, field) */
+       DG_FORM_TET_MM = 2 }; /* tetrahedra stage kernel with both contractions on the matrix cores */
+typedef struct {
+    int32_t stage_form;          /* DG_FORM_*: launches per stage, dg_rhs and dg_profile_steps */
+    int32_t resident;            /* 1: dg_run takes the resident loop in place of launches per stage */
+    int32_t resident_shape;      /* its block shape: 0 a thread per face node with operator rows in
+                                    registers, 1 with operators in LDS, 2 a thread per node, 3 the same
+                                    at 5 blocks per CU; -1 where the grid has no resident loop */
+    int64_t stage_blocks;        /* blocks of a step's final RK4 stage launch */
+    int64_t resident_blocks;     /* blocks of a resident launch, those of learned faces included */
+    int64_t resident_launches;   /* resident launches of dg_run that ran to their end */
+    int64_t resident_aborts;     /* batches handed back to launches per stage: a block waited too long
+                                    for another, or the launch was refused */
+} dg_forms;
+DG_API dg_status dg_get_forms(const dg_context* ctx, dg_forms* forms);
 
 /* Per-kernel device time of `steps` eager RK4 steps measured with HIP events on the
    context's stream: stage_ms[4] (mean per launch of stages 1..4), source_ms, post_ms.
