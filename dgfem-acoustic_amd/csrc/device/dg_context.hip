@@ -140,6 +140,7 @@ struct dg_context {
     int resShape = 0;                  // dgk::kRes*
     int resChunk = 0;                  // steps per launch
     int64_t resLaunches = 0, resAborts = 0;  // launches that ran to their end; batches handed back
+    bool resOff = false;                     // after the first of those
     unsigned char* resMail = nullptr;  // two sets of mailboxes, then outcomes and counts per chunk
     size_t resMailBytes = 0;           //   of one set
     int *resOutcome = nullptr, *resDone = nullptr;
@@ -1129,7 +1130,15 @@ void pickResident(dg_context* c) {
     c->resDone = c->resOutcome + chunks;
 }
 
-bool useResident(const dg_context* c) { return c->resBlocks > 0 && c->resChunk >= kResMinChunk; }
+// A context whose loop handed a batch back launches per stage from then on: what made its blocks wait
+// (another process on the card) tends to last, and every further attempt costs its patience.
+bool useResident(const dg_context* c) { return c->resBlocks > 0 && c->resChunk >= kResMinChunk && !c->resOff; }
+
+// Longest wait of a block for another before a launch is given up, in microseconds. Waits are a few
+// microseconds; a launch whose blocks do not all fit (two processes on one card do not see each other's
+// cooperative launches) would wait for good. Short against what a call takes, long against the
+// dispatch of the last blocks behind other kernels.
+constexpr uint64_t kResPatienceUs = 20000;
 
 template <typename T>
 hipError_t launchChunk(dg_context* c, int chunk, int64_t slot0, int steps, int64_t batch, int integrator, bool resid) {
@@ -1163,7 +1172,7 @@ hipError_t launchChunk(dg_context* c, int chunk, int64_t slot0, int steps, int64
     a.slot0 = slot0;
     a.batchSteps = batch;
     const char* env = std::getenv("DGFEM_RESIDENT_PATIENCE");  // microseconds; 0: no wait at all
-    a.patience = env && env[0] ? std::strtoull(env, nullptr, 10) * 100 : 200000000ull;  // 2 s
+    a.patience = (env && env[0] ? std::strtoull(env, nullptr, 10) : kResPatienceUs) * 100;
     a.dt = static_cast<T>(c->curDt);
     a.steps = steps;
     a.chunk = chunk;
@@ -1734,7 +1743,6 @@ dg_status dg_run(dg_context* c, const dg_run_params* prm, dg_step_fn on_step, dg
         c->curResid = resid ? 1 : 0;
         c->curDt = prm->dt;
         const bool useGraph = c->opt.use_graph != 0;
-        const bool resident = useResident(c);
         auto readyGraphs = [&] {
             if (useGraph && (c->gOne == nullptr || c->gIntegrator != prm->integrator || c->gResid != (resid ? 1 : 0) ||
                              c->gSteps != c->opt.steps_per_graph || c->gDt != prm->dt))
@@ -1750,7 +1758,7 @@ dg_status dg_run(dg_context* c, const dg_run_params* prm, dg_step_fn on_step, dg
                 for (; s < n; ++s) launchStep(c, prm->integrator, resid);
             }
         };
-        if (!resident) readyGraphs();
+        if (!useResident(c)) readyGraphs();
         const int64_t nsteps = static_cast<int64_t>(times.size());
         const int ns = static_cast<int>(c->srcNodes.size());
         const int no = static_cast<int>(c->obsNodes.size());
@@ -1797,7 +1805,7 @@ dg_status dg_run(dg_context* c, const dg_run_params* prm, dg_step_fn on_step, dg
                                n, c->nonfinite, c->srcBase, int64_t(0));
             HIPCHK(hipEventRecord(ev0, c->stream));
             c->sourceFn(c);
-            if (resident) {
+            if (useResident(c)) {
                 outcome.assign(launchResidentBatch(c, n, prm->integrator, resid), dgk::kPending);
                 HIPCHK(hipMemcpyAsync(outcome.data(), c->resOutcome, outcome.size() * sizeof(int), hipMemcpyDeviceToHost,
                                       c->stream));
@@ -1807,6 +1815,7 @@ dg_status dg_run(dg_context* c, const dg_run_params* prm, dg_step_fn on_step, dg
                 c->resLaunches += good;
                 if (good < static_cast<int64_t>(outcome.size())) {
                     ++c->resAborts;
+                    c->resOff = true;
                     // a block waited too long: the state is the one before chunk `good`
                     readyGraphs();
                     hipLaunchKernelGGL(dgk::setCounterKernel, dim3(1), dim3(1), 0, c->stream, c->counter, c->batchSteps, n,

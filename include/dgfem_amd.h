@@ -184,7 +184,9 @@ typedef struct {
     int64_t resident_blocks;     /* blocks of a resident launch, those of learned faces included */
     int64_t resident_launches;   /* resident launches of dg_run that ran to their end */
     int64_t resident_aborts;     /* batches handed back to launches per stage: a block waited too long
-                                    for another, or the launch was refused */
+                                    for another (20 ms, environment DGFEM_RESIDENT_PATIENCE in
+                                    microseconds), or the launch was refused. The context's steps are
+                                    launches per stage from then on (resident 0) */
 } dg_forms;
 DG_API dg_status dg_get_forms(const dg_context* ctx, dg_forms* forms);
 

@@ -1,6 +1,7 @@
 """Which code runs a context's steps (dg_get_forms): the cases of the tests that compare the forms without
 a DGFEM_KERNEL name with other kernels do run them, the resident loop hands no batch of theirs back, and
 the default rules take each form on its side of the line."""
+import numpy as np
 import pytest
 
 import dgfem_amd as dg
@@ -56,8 +57,40 @@ def test_resident_cases_are_resident(dim, order, fields, n, precision, learned, 
 def test_fallback_is_seen(forms, monkeypatch):
     print("case forms fallback", flush=True)
     test_gpu_resident.test_waiting_block_falls_back(dg.DG_MIXED, monkeypatch)
-    assert [f.resident_aborts > 0 for f in forms] == [False, True]
+    assert [f.resident_aborts for f in forms] == [0, 1]
     assert [f.resident_launches for f in forms] == [0, 0]
+
+
+@pytest.mark.parametrize("precision", [dg.DG_FP64, dg.DG_MIXED])
+def test_no_second_attempt(precision, forms, monkeypatch):
+    """Once a batch was handed back, neither the batches after it nor later runs of the context try the
+    resident loop again; another context does."""
+    print(f"case forms no second attempt precision={precision}", flush=True)
+    m = dg.box_mesh(2, 20, 3, jitter=0.1, seed=3)
+    u = np.zeros((4, m.K * m.Np))
+    u[0] = np.exp(-(m.node_coords.reshape(-1, 3) ** 2).sum(1) / 0.1)
+    states = []
+    for patience in ("0", "2000000"):
+        monkeypatch.setenv("DGFEM_RESIDENT_PATIENCE", patience)
+        s = dg.Solver(m.node_coords, m.element_vertices, 3, None, rho0=1.225, c0=340.0, precision=precision)
+        dt = s.info().min_inradius / (340.0 * 7)
+        s.set_state(u)
+        assert s.forms().resident == 1
+        assert s.run(0.0, 39.5 * dt, dt, 9.5 * dt).steps == 40  # 4 batches and a rest
+        f = s.forms()
+        if patience == "0":
+            assert (f.resident, f.resident_launches, f.resident_aborts) == (0, 0, 1)
+            monkeypatch.delenv("DGFEM_RESIDENT_PATIENCE")
+        else:
+            assert f.resident == 1 and f.resident_launches >= 4 and f.resident_aborts == 0
+        s.run_steps(20, dt)
+        g = s.forms()
+        assert g.resident == f.resident and g.resident_aborts == f.resident_aborts
+        assert g.resident_launches == f.resident_launches + f.resident
+        states.append(s.get_state())
+        s.close()
+    tol = test_gpu_resident.TOL[precision]
+    assert 0 < np.linalg.norm(states[0]) and np.linalg.norm(states[0] - states[1]) <= tol * np.linalg.norm(states[1])
 
 
 @pytest.mark.parametrize("integrator", [dg.DG_RK4, dg.DG_EULER])
