@@ -230,7 +230,8 @@ __global__ __launch_bounds__(kBlock, (ResidentShape<DIM, P, NF, T, SHAPE>::kWave
     __shared__ __align__(32) T sN[EB * NFC * 8];  // unit normal, Fscale; h n, h (v0.n) with h = Fscale / 2
     __shared__ __align__(16) T sOps[kOpsN];
     __shared__ double sRed[kBlock / 16][5];
-    __shared__ int sAbort;
+    __shared__ int sAborts[2];  // a thread of the block gave up (learned faces: by epoch, else the first)
+    int& sAbort = sAborts[0];
 
     if (a.chunk > 0 && a.outcome[a.chunk - 1] != kDone) {  // an earlier chunk of the batch was aborted
         if (threadIdx.x == 0) a.outcome[a.chunk] = kAborted;
@@ -245,7 +246,7 @@ __global__ __launch_bounds__(kBlock, (ResidentShape<DIM, P, NF, T, SHAPE>::kWave
 #pragma unroll
     for (int k = 0; k < NF; ++k) none[k] = emptyValue<T>();
     const int nst = a.euler ? 1 : 4;
-    if (tid == 0) sAbort = 0;
+    if (tid < 2) sAborts[tid] = 0;
 
     if (static_cast<int>(blockIdx.x) >= a.blocks) {
         // ---- a block of learned faces: trace in, exterior state out, once per stage ----
@@ -268,7 +269,7 @@ __global__ __launch_bounds__(kBlock, (ResidentShape<DIM, P, NF, T, SHAPE>::kWave
                     const uint64_t t0 = __builtin_amdgcn_s_memrealtime();
                     for (int tries = 1; !arrived<NF>(qm); ++tries) {
                         if ((tries % 64 == 0 || a.patience == 0) && giveUp(outcome, t0, a.patience)) {
-                            sAbort = 1;
+                            sAborts[epoch & 1] = 1;
                             break;
                         }
                         loadMail<NF>(mail, set, fifth, in, qm);
@@ -279,7 +280,9 @@ __global__ __launch_bounds__(kBlock, (ResidentShape<DIM, P, NF, T, SHAPE>::kWave
                     for (int k = 0; k < NF; ++k) qm[k] = T(0);
                 }
                 dgc::closureExterior<DIM, NFP, NF>(w, lds, a.ph, n, qm, qp);
-                if (sAbort) return;  // (set before the barriers inside)
+                // (set before the barriers inside, and not again before those of the next epoch: all
+                // threads read the same here, also when a wave is already polling the next epoch's)
+                if (sAborts[epoch & 1]) return;
                 waitStores();
                 if (mine) storeMail<NF>(mail, set, fifth, out, qp);
             }
