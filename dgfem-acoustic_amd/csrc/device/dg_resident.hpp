@@ -11,7 +11,9 @@
 // in turn). The owner of the exterior value stores it there as soon as its stage is done; the
 // reader polls the mailbox itself, so a trace takes one store and one load and no flag, fence or
 // block-wide wait lies between. An empty mailbox holds kEmpty words (a NaN pattern no arithmetic
-// produces); every word is checked, so the order in which they arrive does not matter. The reader
+// produces); every value is checked, so the order in which they arrive does not matter. Of a double
+// the check looks at the high word only, since a low word may hold any bits: it relies on the aligned
+// 8 bytes of a double becoming visible at once, although they are part of a 16-byte store. The reader
 // empties the mailbox again, and has that store acknowledged before it sends its own next trace
 // of the same face node; the owner writes the same mailbox two epochs later, after it received
 // that trace, so a mailbox is always empty when it is written.
@@ -230,8 +232,7 @@ __global__ __launch_bounds__(kBlock, (ResidentShape<DIM, P, NF, T, SHAPE>::kWave
     __shared__ __align__(32) T sN[EB * NFC * 8];  // unit normal, Fscale; h n, h (v0.n) with h = Fscale / 2
     __shared__ __align__(16) T sOps[kOpsN];
     __shared__ double sRed[kBlock / 16][5];
-    __shared__ int sAborts[2];  // a thread of the block gave up (learned faces: by epoch, else the first)
-    int& sAbort = sAborts[0];
+    __shared__ int sAbort;  // not 0: a thread of the block gave up (learned faces: in epoch sAbort - 1)
 
     if (a.chunk > 0 && a.outcome[a.chunk - 1] != kDone) {  // an earlier chunk of the batch was aborted
         if (threadIdx.x == 0) a.outcome[a.chunk] = kAborted;
@@ -246,7 +247,7 @@ __global__ __launch_bounds__(kBlock, (ResidentShape<DIM, P, NF, T, SHAPE>::kWave
 #pragma unroll
     for (int k = 0; k < NF; ++k) none[k] = emptyValue<T>();
     const int nst = a.euler ? 1 : 4;
-    if (tid < 2) sAborts[tid] = 0;
+    if (tid == 0) sAbort = 0;
 
     if (static_cast<int>(blockIdx.x) >= a.blocks) {
         // ---- a block of learned faces: trace in, exterior state out, once per stage ----
@@ -269,7 +270,7 @@ __global__ __launch_bounds__(kBlock, (ResidentShape<DIM, P, NF, T, SHAPE>::kWave
                     const uint64_t t0 = __builtin_amdgcn_s_memrealtime();
                     for (int tries = 1; !arrived<NF>(qm); ++tries) {
                         if ((tries % 64 == 0 || a.patience == 0) && giveUp(outcome, t0, a.patience)) {
-                            sAborts[epoch & 1] = 1;
+                            sAbort = epoch + 1;
                             break;
                         }
                         loadMail<NF>(mail, set, fifth, in, qm);
@@ -280,9 +281,9 @@ __global__ __launch_bounds__(kBlock, (ResidentShape<DIM, P, NF, T, SHAPE>::kWave
                     for (int k = 0; k < NF; ++k) qm[k] = T(0);
                 }
                 dgc::closureExterior<DIM, NFP, NF>(w, lds, a.ph, n, qm, qp);
-                // (set before the barriers inside, and not again before those of the next epoch: all
-                // threads read the same here, also when a wave is already polling the next epoch's)
-                if (sAborts[epoch & 1]) return;
+                // (this epoch's value is set before the barriers inside, so all threads leave or none:
+                // one already polling for the next epoch may write that epoch's here)
+                if (sAbort == epoch + 1) return;
                 waitStores();
                 if (mine) storeMail<NF>(mail, set, fifth, out, qp);
             }
