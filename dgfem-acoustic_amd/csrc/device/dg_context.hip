@@ -1113,6 +1113,10 @@ void pickResident(dg_context* c) {
     for (int shape = 0; shape < dgk::kResShapes; ++shape) {
         const int eb = dgk::residentElements(c->dim, c->p, shape);
         if (eb == 0) return;
+        // triangles of order 1: the tightest shape's spills cost more than the launches (108,578 elements,
+        // 4 / 5 fields, us per step: 37.5 > 38.3 / 48.1 > 53.3), unless the launches evaluate learned
+        // faces (103,058: 53.4 > 42.2 / 64.8 > 61.3)
+        if (shape == dgk::kResTight && c->dim == 2 && c->p == 1 && c->nLearned == 0) continue;
         n = (c->K + eb - 1) / eb;
         c->resShape = shape;
         c->resGrid = n + (c->nLearned + dgc::kTileFaces - 1) / dgc::kTileFaces;

@@ -89,7 +89,8 @@ struct ResidentArgs {
 //   kResSpread: the same elements per block, operators in LDS: 4 blocks per CU (FP64 tetrahedra and
 //     order 1: 3);
 //   kResDense: as many elements as have their nodes covered, several face nodes per thread;
-//   kResTight: the same in FP32 at 5 blocks per CU.
+//   kResTight: the same in FP32 at 5 blocks per CU (it spills 8 to 76 registers with 4 fields and 37 to
+//     106 with 5).
 // Measured against a launch per stage (us per step, 4 fields, one observer; start > resident):
 //   triangles p=3 mixed: 200 elements 24.4 > 8.6, 8,000 26.6 > 9.6, 18,000 28.8 > 13.7;
 //   FP64 26.5 > 10.5, 31.5 > 14.4, 38.6 > 23.7; p=1 mixed 40,000 25.8 > 12.8;
@@ -97,6 +98,14 @@ struct ResidentArgs {
 //   p=3 mixed: 8,000 38.0 > 24.1, FP64 54.3 > 41.3;
 //   learned walls: triangles p=4 mixed 200 42.0 > 19.6, 20,000 54.7 > 26.5; tetrahedra p=3 mixed
 //   160 45.6 > 22.7, 8,000 56.7 > 29.4.
+// The largest grids of a shape, 4 / 5 fields:
+//   mixed kResDense: triangles p=1 86,528 30.6 > 24.8 / 39.2 > 32.0, p=3 25,538 32.0 > 18.5 / 39.2 > 23.1,
+//   tetrahedra p=3 10,368 45.0 > 27.1 / 55.8 > 37.3;
+//   mixed kResTight: triangles p=2 53,138 35.8 > 30.2 / 46.9 > 41.7, p=3 31,752 35.8 > 27.4 / 46.1 > 37.9,
+//   p=5 15,138 40.0 > 22.6 / 52.4 > 29.6, tetrahedra p=3 13,182 50.6 > 38.7 / 63.3 > 51.9 (triangles of
+//   order 1 lose there: pickResident);
+//   FP64: triangles p=1 31,752 30.1 > 21.8 / 34.9 > 29.4, p=3 21,218 45.4 > 26.1 / 60.1 > 35.4, tetrahedra
+//   p=2 6,000 34.8 > 23.8 / 38.9 > 31.4, p=3 7,986 56.1 > 40.1 / 72.2 > 56.7.
 template <int DIM, int P, int NF, typename T, int SHAPE>
 struct ResidentShape {
     using S = Sizes<DIM, P>;

@@ -117,3 +117,15 @@ def test_default_rules(precision, order, n, form, forms):
     assert s.forms().stage_form == form
     assert s.forms().resident == 0
     s.close()
+
+
+@pytest.mark.parametrize("fields", [4, 5])
+@pytest.mark.parametrize("n,walls,shape", [(208, "rigid", 2), (222, "rigid", -1), (233, "rigid", -1), (222, "learned", 3)])
+def test_order_1_triangles_at_5_blocks_per_cu(n, walls, shape, fields, forms):
+    print(f"case forms order 1 n={n} walls={walls} fields={fields}", flush=True)
+    m = dg.box_mesh(2, n, 1)
+    bc = dg.resolve_bc_sides(m, [(0xF, dg.DG_BC_LEARNED if walls == "learned" else dg.DG_BC_REFLECTING)])
+    s = dg.Solver(m.node_coords, m.element_vertices, 1, bc, fields=dg.DG_FIELDS_LEE5 if fields == 5 else dg.DG_FIELDS_REF4,
+                  precision=dg.DG_MIXED)
+    assert (s.forms().resident_shape, s.forms().resident) == (shape, int(shape >= 0))
+    s.close()
