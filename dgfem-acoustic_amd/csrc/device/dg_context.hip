@@ -1191,6 +1191,8 @@ hipError_t launchChunk(dg_context* c, int chunk, int64_t slot0, int steps, int64
 int launchResidentBatch(dg_context* c, int64_t n, int integrator, bool resid) {
     const int chunks = static_cast<int>((n + c->resChunk - 1) / c->resChunk);
     const int64_t ns = static_cast<int64_t>(c->srcNodes.size());
+    const char* env = std::getenv("DGFEM_RESIDENT_LAUNCHES");  // (tests) launches per batch before one is refused
+    const int most = env && env[0] ? std::atoi(env) : chunks;
     if (ns > 0)
         hipLaunchKernelGGL(dgk::residentSourceKernel, dim3(static_cast<unsigned>((n * ns + 255) / 256)), dim3(256), 0,
                            c->stream, sourceArgs(c), n, c->dSrcVal);
@@ -1201,8 +1203,8 @@ int launchResidentBatch(dg_context* c, int64_t n, int integrator, bool resid) {
         hipLaunchKernelGGL(dgk::residentResetKernel, dim3(static_cast<unsigned>((clear + 255) / 256)), dim3(256), 0,
                            c->stream, reinterpret_cast<uint4*>(c->resMail), words, c->resOutcome, c->resDone,
                            k == 0 ? chunks : 0);
-        if ((c->precision == DG_FP64 ? launchChunk<double>(c, k, s0, steps, n, integrator, resid)
-                                     : launchChunk<float>(c, k, s0, steps, n, integrator, resid)) != hipSuccess) {
+        if (k >= most || (c->precision == DG_FP64 ? launchChunk<double>(c, k, s0, steps, n, integrator, resid)
+                                                  : launchChunk<float>(c, k, s0, steps, n, integrator, resid)) != hipSuccess) {
             (void)hipGetLastError();  // not launched: its outcome stays kPending
             break;
         }

@@ -1835,10 +1835,11 @@ __global__ __launch_bounds__(kPostBlock) void postKernel(PostArgs p, SourceArgs 
 
 [[maybe_unused]] static __global__ void setCounterKernel(int64_t* counter, int64_t* batchSteps, int64_t nsteps, int* flag,
                                                          int64_t* srcBase, int64_t first) {
-    // `first` > 0: the batch goes on at that step (what earlier steps reported stays)
+    // `first` > 0: the batch goes on at that step. What earlier steps reported stays, what a given-up
+    // launch of later ones reported goes: its blocks were not all as far.
     *counter = first;
     *batchSteps = nsteps;
-    if (first == 0) flag[0] = -1;
+    if (first == 0 || flag[0] >= first) flag[0] = -1;
     flag[1] = 0;
     *srcBase = first;
 }
