@@ -186,6 +186,9 @@ constexpr int kClosureBlock = 256;
 constexpr int kFrag1 = 4 * 64, kFrag2 = 4 * 2 * 64, kFrag3 = 2 * 64;
 constexpr int kNetWords = kFrag1 + kFrag2 + kFrag3 + (64 + 64 + 16) / 4;  // of 16 bytes
 
+// An infinite weight of a hidden layer becomes the largest finite one: its products with the small terms
+// of an activation, which are zero where the first holds it exactly, would be NaN, while the sum is
+// infinite and its tanh +-1 either way.
 inline void packClosure(int nin, int nout, const uint16_t* w, uint32_t* out) {
     const uint16_t *w1 = w, *b1 = w1 + kH * nin, *w2 = b1 + kH, *b2 = w2 + kH * kH, *w3 = b2 + kH, *b3 = w3 + nout * kH;
     uint16_t* h = reinterpret_cast<uint16_t*>(out);
@@ -194,6 +197,7 @@ inline void packClosure(int nin, int nout, const uint16_t* w, uint32_t* out) {
             for (int j = 0; j < 8; ++j, ++h) {
                 const int r = row0 + lane % 16, c = col0 + 8 * (lane / 16) + j;
                 *h = r < rows && c < cols ? m[r * cols + c] : uint16_t(0);
+                if (m != w3 && (*h & 0x7fff) == 0x7f80) --*h;
             }
     };
     for (int t = 0; t < 4; ++t) put(w1, kH, nin, 16 * t, 0);
