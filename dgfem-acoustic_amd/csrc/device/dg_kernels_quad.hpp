@@ -1,4 +1,4 @@
-// Stage kernel with a lane per (element, field): FP32, 4 fields (mixed precision).
+// Stage kernel with a lane per (element, field): tetrahedra, FP32, 4 fields (mixed precision).
 //
 // A wave owns 16 elements; lane 4 b + f holds field f of element b, all nodes of it in registers.
 // v_mfma_f32_4x4x1_16b_f32 multiplies 16 independent 4 x 1 by 1 x 4 blocks: with block = element and
@@ -37,8 +37,9 @@
 
 namespace dgk {
 
-template <int DIM, int P>
+template <int P>
 struct QuadShape {
+    static constexpr int DIM = 3;
     using S = Sizes<DIM, P>;
     static constexpr int NP = S::NP, NFP = S::NFP, NFC = S::NFC, NFT = S::NFT;
     static constexpr int kGroup = 16;                       // elements per wave
@@ -52,44 +53,32 @@ struct QuadShape {
     static constexpr int TW = (NFP + 3) / 4;                // words of a row of node bytes
 };
 
-// Canonical lattice index of a barycentric tuple (loops l_DIM outer .. l_1 inner).
-template <int DIM, int P>
+// Canonical lattice index of a barycentric tuple (loops l_3 outer .. l_1 inner).
+template <int P>
 constexpr int latticeIndex(int b1, int b2, int b3) {
     int n = 0;
-    if (DIM == 2) {
-        for (int j = 0; j <= P; ++j)
-            for (int i = 0; i <= P - j; ++i, ++n)
-                if (i == b1 && j == b2) return n;
-    } else {
-        for (int k = 0; k <= P; ++k)
-            for (int j = 0; j <= P - k; ++j)
-                for (int i = 0; i <= P - j - k; ++i, ++n)
-                    if (i == b1 && j == b2 && k == b3) return n;
-    }
+    for (int k = 0; k <= P; ++k)
+        for (int j = 0; j <= P - k; ++j)
+            for (int i = 0; i <= P - j - k; ++i, ++n)
+                if (i == b1 && j == b2 && k == b3) return n;
     return -1;
 }
 
 // Element node of face node a of local face f (the table dg::RefElement::fmask as a constant, so
 // that it selects registers; launchStageQuad's caller checks it against the table).
-template <int DIM, int P>
+template <int P>
 constexpr int faceNode(int f, int a) {
-    constexpr int v2[3][2] = {{0, 1}, {1, 2}, {2, 0}};
-    constexpr int v3[4][3] = {{0, 2, 1}, {0, 1, 3}, {0, 3, 2}, {3, 1, 2}};
+    constexpr int v[4][3] = {{0, 2, 1}, {0, 1, 3}, {0, 3, 2}, {3, 1, 2}};
     int b[4] = {0, 0, 0, 0};
-    if (DIM == 2) {
-        b[v2[f][0]] = P - a;
-        b[v2[f][1]] = a;
-    } else {
-        int n = 0;
-        for (int j = 0; j <= P; ++j)
-            for (int i = 0; i <= P - j; ++i, ++n)
-                if (n == a) {
-                    b[v3[f][0]] = P - i - j;
-                    b[v3[f][1]] = i;
-                    b[v3[f][2]] = j;
-                }
-    }
-    return latticeIndex<DIM, P>(b[1], b[2], b[3]);
+    int n = 0;
+    for (int j = 0; j <= P; ++j)
+        for (int i = 0; i <= P - j; ++i, ++n)
+            if (n == a) {
+                b[v[f][0]] = P - i - j;
+                b[v[f][1]] = i;
+                b[v[f][2]] = j;
+            }
+    return latticeIndex<P>(b[1], b[2], b[3]);
 }
 
 template <int N, typename Fn, int... I>
@@ -119,9 +108,10 @@ __device__ inline mf4 quadMma(float a, float b, mf4 c) {
     return __builtin_amdgcn_mfma_f32_4x4x1f32(a, b, c, 4, ABID, 0);
 }
 
-template <int DIM, int P, bool COMP, int MODE>
+template <int P, int MODE>
 __global__ __launch_bounds__(256, (MODE == kModeFinal || MODE == kModeEuler ? 2 : 3)) void stageKernelQuad(StageArgs<float> a, int64_t nGroups) {
-    using Q = QuadShape<DIM, P>;
+    using Q = QuadShape<P>;
+    constexpr int DIM = Q::DIM;
     using L = OpLayout<DIM, P>;
     constexpr int NP = Q::NP, NFP = Q::NFP, NFC = Q::NFC, RG = Q::RG, ES = Q::ES, NCH = Q::NCH, G = Q::kGroup;
     constexpr int JJ = DIM * DIM, TW = Q::TW, NPERM = Sizes<DIM, P>::NPERM;
@@ -153,15 +143,15 @@ __global__ __launch_bounds__(256, (MODE == kModeFinal || MODE == kModeEuler ? 2 
     const int64_t g0 = wi * nGroups / nw, g1 = (wi + 1) * nGroups / nw;
     const char* const qbase = reinterpret_cast<const char*>(a.qin);
 
-    // what a group needs first, loaded a group ahead
-    struct Ahead {
+    // what a group needs first (its loads one behind another; loading them a group ahead measured no gain)
+    struct Group {
         float q[NCH][4];
         int nb[NFC];
-        uint32_t cd[NFC == 4 ? 1 : NFC];
+        uint32_t cd;  // of the 4 faces
         float fg[NFC];  // h = Fscale / 2: h (v0.n) on lane 0, h n on lanes 1..3 (rounded once from FP64)
         float J[DIM];   // dxi_r/dx of the lane's direction
     };
-    auto loadAhead = [&](int64_t grp, Ahead& n) __attribute__((always_inline)) {
+    auto loadGroup = [&](int64_t grp, Group& n) __attribute__((always_inline)) {
         int lane = tid & 63;
         asm volatile("" : "+v"(lane));
         const int el = lane >> 2, f = lane & 3;
@@ -176,31 +166,26 @@ __global__ __launch_bounds__(256, (MODE == kModeFinal || MODE == kModeEuler ? 2 
         }
         const int32_t* nbg = a.nbr + e0 * NFC;
         const uint8_t* cdg = a.code + e0 * NFC;
-        if constexpr (NFC == 4) {
-            const int4 v = reinterpret_cast<const int4*>(nbg)[e];
-            n.nb[0] = v.x, n.nb[1] = v.y, n.nb[2] = v.z, n.nb[3] = v.w;
-            n.cd[0] = reinterpret_cast<const uint32_t*>(cdg)[e];
-        } else {
-#pragma unroll
-            for (int k = 0; k < NFC; ++k) n.nb[k] = nbg[e * NFC + k], n.cd[k] = cdg[e * NFC + k];
-        }
+        const int4 v = reinterpret_cast<const int4*>(nbg)[e];
+        n.nb[0] = v.x, n.nb[1] = v.y, n.nb[2] = v.z, n.nb[3] = v.w;
+        n.cd = reinterpret_cast<const uint32_t*>(cdg)[e];
         const float* fgg = a.fgeo + e0 * NFC * 4;
 #pragma unroll
         for (int k = 0; k < NFC; ++k) n.fg[k] = fgg[(e * NFC + k) * 4 + ((f + 3) & 3)];
         const float* gg = a.geo + e0 * JJ;
 #pragma unroll
-        for (int r = 0; r < DIM; ++r) n.J[r] = gg[e * JJ + r * DIM + (f >= 1 && f <= DIM ? f - 1 : 0)];
+        for (int r = 0; r < DIM; ++r) n.J[r] = gg[e * JJ + r * DIM + (f >= 1 ? f - 1 : 0)];
     };
     for (int64_t grp = g0; grp < g1; ++grp) {
-        Ahead cur;
-        loadAhead(grp, cur);
+        Group cur;
+        loadGroup(grp, cur);
         // (opaque, so that what follows from the lane is not kept in registers over the loop)
         int lane = tid & 63;
         asm volatile("" : "+v"(lane));
         const int el = lane >> 2, f = lane & 3;
         const float v0l = f == 0 ? 0.0f : f == 1 ? ph.v0[0] : f == 2 ? ph.v0[1] : ph.v0[2];
         const float pl = f == 0 ? 1.0f : 0.0f;  // 1 on the pressure's lane
-        const bool dirLane = f >= 1 && f <= DIM;
+        const bool dirLane = f >= 1;
         const int64_t e0 = grp * G;
         const int nE = static_cast<int>((a.K - e0) < G ? (a.K - e0) : G);
         const int64_t e = e0 + (el < nE ? el : 0);  // this lane's element (clamped)
@@ -209,7 +194,7 @@ __global__ __launch_bounds__(256, (MODE == kModeFinal || MODE == kModeEuler ? 2 
 #pragma unroll
         for (int k = 0; k < NFC; ++k) {
             nb[k] = cur.nb[k];
-            cd[k] = NFC == 4 ? (cur.cd[0] >> (8 * k)) & 0xff : cur.cd[NFC == 4 ? 0 : k];
+            cd[k] = (cur.cd >> (8 * k)) & 0xff;
             fg[k] = cur.fg[k];
         }
 #pragma unroll
@@ -319,14 +304,14 @@ __global__ __launch_bounds__(256, (MODE == kModeFinal || MODE == kModeEuler ? 2 
                     wC = nl * ph.irho0 * fs;
                 } else {
                     const float ac = 0.25f * fs * (ph.c0 + vn0), vl = vn0 < 0.0f ? 0.0f : -0.25f * fs * vn0;
-                    wA = f == 0 ? ac : (DIM == 3 || f < 3) ? -vl : 0.0f;
+                    wA = f == 0 ? ac : -vl;
                     wB = f == 0 ? ph.c0 * ph.rho0 * ac : (ac + vl) * nl;
                     wC = nl * ac * ph.irc0;
                 }
             }
             float pi[NFP];
             staticFor<NFP>([&](auto xc) {
-                constexpr int x = decltype(xc)::value, own = faceNode<DIM, P>(k, x), fa = k * NFP + x;
+                constexpr int x = decltype(xc)::value, own = faceNode<P>(k, x), fa = k * NFP + x;
                 const float qm = q[own], qe = qp[fa];
                 const float qs = qm + s * qe;
                 const float nv = quadSum(gl * qs);
@@ -377,25 +362,20 @@ __global__ __launch_bounds__(256, (MODE == kModeFinal || MODE == kModeEuler ? 2 
                 storeNodeNT<4>(a.acc + gb + x * 4, accn);
                 storeNode<4>(a.qout + gb + x * 4, qn);
             } else {
-                float plo[4] = {0, 0, 0, 0}, ps[4], unew[4], lnew[4];
-                if constexpr (COMP) loadNodeNT<4>(a.ulo + gb + x * 4, plo);
+                float plo[4], ps[4], unew[4], lnew[4];
+                loadNodeNT<4>(a.ulo + gb + x * 4, plo);
                 if (a.snap) loadNodeNT<4>(a.snap + gb + x * 4, ps);
 #pragma unroll
                 for (int k = 0; k < 4; ++k) {
                     const float kk = dt * rhs[k];
                     const float delta = (MODE == kModeFinal) ? (pacc[c][k] + kk) / 6.0f : kk;
-                    if constexpr (COMP) {
-                        float s_, e_, t_, e2;
-                        twoSum(plo[k], delta, t_, e2);
-                        twoSum(pu[c][k], t_, s_, e_);
-                        twoSum(s_, e_ + e2, unew[k], lnew[k]);
-                    } else {
-                        unew[k] = pu[c][k] + delta;
-                        lnew[k] = 0.0f;
-                    }
+                    float s_, e_, t_, e2;
+                    twoSum(plo[k], delta, t_, e2);
+                    twoSum(pu[c][k], t_, s_, e_);
+                    twoSum(s_, e_ + e2, unew[k], lnew[k]);
                 }
                 storeNodeNT<4>(a.uout + gb + x * 4, unew);
-                if constexpr (COMP) storeNodeNT<4>(a.ulo + gb + x * 4, lnew);
+                storeNodeNT<4>(a.ulo + gb + x * 4, lnew);
                 if (!allFinite<4>(unew)) a.stateBad[0] = 1;
                 if (a.snap) {
                     double d[4];

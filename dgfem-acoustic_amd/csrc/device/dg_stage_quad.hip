@@ -15,11 +15,11 @@ namespace {
 using Kernel = void (*)(StageArgs<float>, int64_t);
 Kernel kernelOf(int mode) {
     switch (mode) {
-        case kModeFirst: return &stageKernelQuad<3, 3, true, kModeFirst>;
-        case kModeMid: return &stageKernelQuad<3, 3, true, kModeMid>;
-        case kModeFinal: return &stageKernelQuad<3, 3, true, kModeFinal>;
-        case kModeEuler: return &stageKernelQuad<3, 3, true, kModeEuler>;
-        default: return &stageKernelQuad<3, 3, true, kModeRHS>;
+        case kModeFirst: return &stageKernelQuad<3, kModeFirst>;
+        case kModeMid: return &stageKernelQuad<3, kModeMid>;
+        case kModeFinal: return &stageKernelQuad<3, kModeFinal>;
+        case kModeEuler: return &stageKernelQuad<3, kModeEuler>;
+        default: return &stageKernelQuad<3, kModeRHS>;
     }
 }
 
@@ -27,12 +27,12 @@ Kernel kernelOf(int mode) {
 
 bool buildQuadFrag(int dim, int p, const double* Dw, const double* LIFT, const int32_t* fmask, std::vector<double>& frag) {
     if (dim != 3 || p != 3) return false;
-    constexpr int DIM = 3, P = 3;
-    using Q = QuadShape<DIM, P>;
+    constexpr int P = 3;
+    using Q = QuadShape<P>;
     bool same = true;
     staticFor<Q::NFC>([&](auto fc) {
         staticFor<Q::NFP>([&](auto ac) {
-            constexpr int f = decltype(fc)::value, a = decltype(ac)::value, n = faceNode<DIM, P>(f, a);
+            constexpr int f = decltype(fc)::value, a = decltype(ac)::value, n = faceNode<P>(f, a);
             same = same && fmask[f * Q::NFP + a] == n;
         });
     });
@@ -45,8 +45,8 @@ bool buildQuadFrag(int dim, int p, const double* Dw, const double* LIFT, const i
     };
     for (int g = 0; g < Q::RG; ++g)
         for (int j = 0; j < Q::NP; ++j)
-            for (int r = 0; r < DIM; ++r)
-                put(0, (g * Q::NP + j) * DIM + r, g,
+            for (int r = 0; r < Q::DIM; ++r)
+                put(0, (g * Q::NP + j) * Q::DIM + r, g,
                     [&](int i) { return Dw[(static_cast<size_t>(r) * Q::NP + i) * Q::NP + j]; });
     for (int fa = 0; fa < Q::NFT; ++fa)
         for (int g = 0; g < Q::RG; ++g)
