@@ -173,9 +173,10 @@ __device__ inline void mlpForwardWave(const float* net, const float* sx, float* 
 // the latency of the chain (three products of 3-6 instructions, two tanh, three exchanges through
 // LDS), so the weights are registers of their lanes. One wave evaluating 4 or 8 faces with a lane per
 // hidden unit and the weights in LDS took 7.2 us (400 faces, order 4 triangles) and 12.1 us
-// (6,912 faces, order 3 tetrahedra) per launch; this takes 4.7 and 6.5, and is as exact or more
-// (FP64 runs with a random network, 100 steps, against 64 bits: 1.5e-10 and 1.9e-10; 3.2e-10 and
-// 5.1e-10 with the wave-per-face kernel).
+// (6,912 faces, order 3 tetrahedra) per launch; this takes 4.7 and 6.5. Mixed-precision states are as
+// far from 64 bits with either (2.4e-7 and 3.4e-7); the network's own rounding, seen by itself when
+// FP64 states were stepped with it for 100 steps, is half as large (1.5e-10 and 1.9e-10 against 3.2e-10
+// and 5.1e-10). FP64 contexts use closureWaveKernel all the same (see there).
 
 constexpr int kTileFaces = 16;
 constexpr int kClosureBlock = 256;

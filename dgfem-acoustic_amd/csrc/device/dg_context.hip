@@ -990,7 +990,12 @@ void launchStepForked(dg_context* c, bool resid, int s) {
 // with a source and two observers breaks even with it (the end-of-step kernel's ~19 µs hidden,
 // about as much added), and a 1,536-block 2D grid ran 39% slower per step. It is kept for large
 // grids, where the end-of-step kernel grows with the residual partials and the observer and
-// source tables while the branch's cost does not. DGFEM_POST_BRANCH = 0 | 1 overrides the rule.
+// source tables while the branch's cost does not. The blocks counted are those of the thread-per-node
+// variant, also where the lane-per-field or the tetrahedra matrix-core kernel runs in its place: with
+// these it makes no difference of more than 1.6% either way (us per step without and with it: 196,608
+// tetrahedra of order 3 332 and 331, with learned walls 358 and 362-364, 355,914 576 and 579; order 5
+// FP64, 24,576: 464 and 463; order 4 FP64, 63,888: 468 and 468, mixed 285 and 286, 162,000: 645 and 641).
+// DGFEM_POST_BRANCH = 0 | 1 overrides the rule.
 constexpr int64_t kBranchMinBlocks = 4096;
 
 // Whether some observer node is also a source node, from the host definitions (the same test
@@ -1074,8 +1079,9 @@ void pickQuad(dg_context* c, const dg::RefElement& R) {
 //   mixed order 4: 4,374 56 > 59 / 64 > 70; 10,368 91 > 81 / 106 > 99; 162,000 862 > 636 / 1080 > 865
 // Not built: order 3 (20 of 32 rows used: broke even in FP64), order 2 (slower), and order 5 in mixed
 // precision, where it is faster than the split-BF16 kernel (48,000 elements 508 > 459) but its error
-// against FP64 larger (5 fields, 150 steps: 4.0e-7 against 2.5e-7; order 4, against the thread-per-node
-// kernel: 2.60e-7 and 2.65e-7). DGFEM_TET_MM=1 takes it at any size, =0 never.
+// against FP64 larger (5 fields, 150 steps: 4.0e-7 against 2.5e-7). At order 4 the mean error of ten runs
+// of 100 steps is 2.84e-7 with the thread-per-node kernel and 2.80e-7 with this one (single runs 3.7%
+// less to 0.4% more). DGFEM_TET_MM=1 takes it at any size, =0 never.
 int64_t tetMMFrom(const dg_context* c) {
     return c->precision == DG_MIXED ? 10000 : c->p == 5 ? 2048 : 6000;
 }

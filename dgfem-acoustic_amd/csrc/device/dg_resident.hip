@@ -75,7 +75,8 @@ int residentBlocksPerCu(int dim, int p, int nf, bool fp64, int shape) {
         hipFuncGetAttributes(&attr, f) != hipSuccess)
         return 0;
     // the LDS of a block is allocated in units the occupancy query does not round to: 5 blocks of
-    // 32,504 bytes fit the 160 KB of a CU by division but were not resident together
+    // 32,504 bytes fit the 160 KB of a CU by division but were not resident together. A margin of 2 KB
+    // per block covers the rounding without knowledge of the unit.
     const int lds = (160 * 1024) / (static_cast<int>(attr.sharedSizeBytes) + 2048);
     return n < lds ? n : lds;
 }
