@@ -141,6 +141,7 @@ struct dg_context {
     int resChunk = 0;                  // steps per launch
     int64_t resLaunches = 0, resAborts = 0;  // launches that ran to their end; batches handed back
     bool resOff = false;                     // after the first of those
+    int resShort = 0;                        // short batches since graphs were last current
     unsigned char* resMail = nullptr;  // two sets of mailboxes, then outcomes and counts per chunk
     size_t resMailBytes = 0;           //   of one set
     int *resOutcome = nullptr, *resDone = nullptr;
@@ -1144,6 +1145,16 @@ void pickResident(dg_context* c) {
 // (another process on the card) tends to last, and every further attempt costs its patience.
 bool useResident(const dg_context* c) { return c->resBlocks > 0 && c->resChunk >= kResMinChunk && !c->resOff; }
 
+// Batches of fewer steps are launched per stage: a resident launch costs 50-60 us before its first step
+// (mailboxes emptied, state and operators loaded, outcome read back). us per call, launches > loop, RK4
+// and forward Euler: 18,432 triangles p=3 mixed n=1 98 > 155 / 86 > 146, n=3 168 > 175 / 129 > 151, n=5
+// 236 > 201 / 174 > 159; 80,000 p=1 n=3 174 > 215 / 133 > 159, n=5 246 > 262 / 180 > 170, n=6 279 > 285 /
+// 202 > 174; 7,986 tetrahedra p=3 mixed n=3 206 > 231 / 147 > 180, n=5 300 > 276 / 202 > 195.
+// Launches need captured graphs, 1 ms for every change of dt or integrator: a context whose other
+// batches are resident captures them with the 16th short batch, when the loop has cost as much.
+constexpr int64_t kResMinSteps = 6;
+constexpr int kResShortBatches = 16;
+
 // Longest wait of a block for another before a launch is given up, in microseconds. Waits are a few
 // microseconds; a launch whose blocks do not all fit (two processes on one card do not see each other's
 // cooperative launches) would wait for good. Short against what a call takes, long against the
@@ -1755,10 +1766,19 @@ dg_status dg_run(dg_context* c, const dg_run_params* prm, dg_step_fn on_step, dg
         c->curResid = resid ? 1 : 0;
         c->curDt = prm->dt;
         const bool useGraph = c->opt.use_graph != 0;
+        auto graphsCurrent = [&] {
+            return !useGraph || (c->gOne != nullptr && c->gIntegrator == prm->integrator && c->gResid == (resid ? 1 : 0) &&
+                                 c->gSteps == c->opt.steps_per_graph && c->gDt == prm->dt);
+        };
         auto readyGraphs = [&] {
-            if (useGraph && (c->gOne == nullptr || c->gIntegrator != prm->integrator || c->gResid != (resid ? 1 : 0) ||
-                             c->gSteps != c->opt.steps_per_graph || c->gDt != prm->dt))
-                captureGraphs(c, prm->integrator, resid, c->opt.steps_per_graph), c->gDt = prm->dt;
+            if (!graphsCurrent()) captureGraphs(c, prm->integrator, resid, c->opt.steps_per_graph), c->gDt = prm->dt;
+            c->resShort = 0;
+        };
+        // whether a batch of n steps runs in the resident loop (else the graphs are ready)
+        auto residentBatch = [&](int64_t n) {
+            if (useResident(c) && (n >= kResMinSteps || (!graphsCurrent() && ++c->resShort < kResShortBatches))) return true;
+            readyGraphs();
+            return false;
         };
         // steps s .. n-1 of a batch, launched kernel by kernel
         auto launchSteps = [&](int64_t s, int64_t n) {
@@ -1786,6 +1806,7 @@ dg_status dg_run(dg_context* c, const dg_run_params* prm, dg_step_fn on_step, dg
             int64_t end = done + 1;
             while (end < nsteps && !isSave[end] && end - done < c->ringSlots) ++end;
             const int64_t n = end - done;
+            const bool resident = residentBatch(n);
             if (isSave[done]) {
                 HIPCHK(hipMemcpyAsync(c->snap, c->u, stateN * c->tsize, hipMemcpyDeviceToDevice, c->stream));
                 if (on_save) {
@@ -1817,7 +1838,7 @@ dg_status dg_run(dg_context* c, const dg_run_params* prm, dg_step_fn on_step, dg
                                n, c->nonfinite, c->srcBase, int64_t(0));
             HIPCHK(hipEventRecord(ev0, c->stream));
             c->sourceFn(c);
-            if (useResident(c)) {
+            if (resident) {
                 outcome.assign(launchResidentBatch(c, n, prm->integrator, resid), dgk::kPending);
                 HIPCHK(hipMemcpyAsync(outcome.data(), c->resOutcome, outcome.size() * sizeof(int), hipMemcpyDeviceToHost,
                                       c->stream));
