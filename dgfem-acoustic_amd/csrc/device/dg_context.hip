@@ -141,7 +141,7 @@ struct dg_context {
     int resChunk = 0;                  // steps per launch
     int64_t resLaunches = 0, resAborts = 0;  // launches that ran to their end; batches handed back
     bool resOff = false;                     // after the first of those
-    int resShort = 0;                        // short batches since graphs were last current
+    int resShort = 0;                        // short batches launched without graphs
     unsigned char* resMail = nullptr;  // two sets of mailboxes, then outcomes and counts per chunk
     size_t resMailBytes = 0;           //   of one set
     int *resOutcome = nullptr, *resDone = nullptr;
@@ -1150,8 +1150,9 @@ bool useResident(const dg_context* c) { return c->resBlocks > 0 && c->resChunk >
 // and forward Euler: 18,432 triangles p=3 mixed n=1 98 > 155 / 86 > 146, n=3 168 > 175 / 129 > 151, n=5
 // 236 > 201 / 174 > 159; 80,000 p=1 n=3 174 > 215 / 133 > 159, n=5 246 > 262 / 180 > 170, n=6 279 > 285 /
 // 202 > 174; 7,986 tetrahedra p=3 mixed n=3 206 > 231 / 147 > 180, n=5 300 > 276 / 202 > 195.
-// Launches need captured graphs, 1 ms for every change of dt or integrator: a context whose other
-// batches are resident captures them with the 16th short batch, when the loop has cost as much.
+// The line is on the steps alone, so that a call does the same whatever came before it. Captured graphs
+// take 1 ms for every change of dt or integrator: a context whose other batches are resident launches
+// its short ones kernel by kernel (the same bits) until the 16th.
 constexpr int64_t kResMinSteps = 6;
 constexpr int kResShortBatches = 16;
 
@@ -1774,15 +1775,9 @@ dg_status dg_run(dg_context* c, const dg_run_params* prm, dg_step_fn on_step, dg
             if (!graphsCurrent()) captureGraphs(c, prm->integrator, resid, c->opt.steps_per_graph), c->gDt = prm->dt;
             c->resShort = 0;
         };
-        // whether a batch of n steps runs in the resident loop (else the graphs are ready)
-        auto residentBatch = [&](int64_t n) {
-            if (useResident(c) && (n >= kResMinSteps || (!graphsCurrent() && ++c->resShort < kResShortBatches))) return true;
-            readyGraphs();
-            return false;
-        };
         // steps s .. n-1 of a batch, launched kernel by kernel
-        auto launchSteps = [&](int64_t s, int64_t n) {
-            if (useGraph) {
+        auto launchSteps = [&](int64_t s, int64_t n, bool graphs) {
+            if (graphs) {
                 if (c->gMulti)
                     for (; s + c->gSteps <= n; s += c->gSteps) HIPCHK(hipGraphLaunch(c->gMulti, c->stream));
                 for (; s < n; ++s) HIPCHK(hipGraphLaunch(c->gOne, c->stream));
@@ -1806,7 +1801,10 @@ dg_status dg_run(dg_context* c, const dg_run_params* prm, dg_step_fn on_step, dg
             int64_t end = done + 1;
             while (end < nsteps && !isSave[end] && end - done < c->ringSlots) ++end;
             const int64_t n = end - done;
-            const bool resident = residentBatch(n);
+            const bool resident = useResident(c) && n >= kResMinSteps;
+            const bool graphs = useGraph && !resident &&
+                                (!useResident(c) || graphsCurrent() || ++c->resShort >= kResShortBatches);
+            if (graphs) readyGraphs();
             if (isSave[done]) {
                 HIPCHK(hipMemcpyAsync(c->snap, c->u, stateN * c->tsize, hipMemcpyDeviceToDevice, c->stream));
                 if (on_save) {
@@ -1853,10 +1851,10 @@ dg_status dg_run(dg_context* c, const dg_run_params* prm, dg_step_fn on_step, dg
                     readyGraphs();
                     hipLaunchKernelGGL(dgk::setCounterKernel, dim3(1), dim3(1), 0, c->stream, c->counter, c->batchSteps, n,
                                        c->nonfinite, c->srcBase, good * c->resChunk);
-                    launchSteps(good * c->resChunk, n);
+                    launchSteps(good * c->resChunk, n, useGraph);
                 }
             } else {
-                launchSteps(0, n);
+                launchSteps(0, n, graphs);
             }
             HIPCHK(hipGetLastError());
             HIPCHK(hipEventRecord(ev1, c->stream));

@@ -177,7 +177,7 @@ enum { DG_FORM_KERNEL = 0,   /* the kernel dg_info.stage_kernel names */
 typedef struct {
     int32_t stage_form;          /* DG_FORM_*: launches per stage, dg_rhs and dg_profile_steps */
     int32_t resident;            /* 1: dg_run takes the resident loop in place of launches per stage
-                                    (batches of at least 6 steps, shorter ones now and then) */
+                                    (batches of at least 6 steps) */
     int32_t resident_shape;      /* its block shape: 0 a thread per face node with operator rows in
                                     registers, 1 with operators in LDS, 2 a thread per node, 3 the same
                                     at 5 blocks per CU; -1 where the grid has no resident loop */

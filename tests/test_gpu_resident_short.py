@@ -1,5 +1,5 @@
 """Short batches (calls of few steps, saves every few steps) of a grid that has the resident loop: launched
-per stage, once the graphs for it are worth capturing; the loop still takes the longer ones."""
+per stage, kernel by kernel at first and captured later; the loop still takes the longer ones."""
 import numpy as np
 import pytest
 
@@ -52,9 +52,34 @@ def test_short_batches(precision, integrator, use_graph, monkeypatch):
         counts.append(seen)
         s.close()
     assert counts[0] == [0] * 28
-    if use_graph:  # the 16th batch captures; a new dt counts anew
-        assert counts[1] == list(range(1, 16)) + [15] * 5 + [16] * 4 + [17, 17, 18, 19]
-    else:  # nothing to capture
-        assert counts[1] == [0] * 20 + [1] * 4 + [2] * 4
+    assert counts[1] == [0] * 20 + [1] * 4 + [2] * 4
     # 107 steps of at most an eighth of the bar's
     test_gpu_resident._close(*out[::-1], test_gpu_resident.TOL[precision])
+
+
+@pytest.mark.parametrize("precision", [dg.DG_FP64, dg.DG_MIXED])
+@pytest.mark.parametrize("steps", [1, 5, 6])
+def test_same_call_same_bits(precision, steps, monkeypatch):
+    """A call from the same state gives the same bits each time: the first, which captures nothing, those
+    after the graphs are captured, with and without the resident loop's calls of another length between."""
+    print(f"case resident same call precision={precision} steps={steps}", flush=True)
+    monkeypatch.delenv("DGFEM_RESIDENT", raising=False)
+    m = dg.box_mesh(2, 12, 3, jitter=0.1, seed=2)
+    X = m.node_coords.reshape(-1, 3)
+    u = np.zeros((4, len(X)))
+    u[0] = np.exp(-(X ** 2).sum(1) / 0.1)
+    s = dg.Solver(m.node_coords, m.element_vertices, 3, None, rho0=1.225, c0=340.0, precision=precision)
+    dt = s.info().min_inradius / (340.0 * 7)
+    s.add_observer(0.4, 0.3, 0.0, 0.3)
+    first = None
+    for k in range(24):
+        if k % 5 == 4:
+            s.run_steps(20, dt)
+        s.set_state(u)
+        r = s.run_steps(steps, dt)
+        got = s.get_state(), r.residuals, r.observers
+        if first is None:
+            first = got
+        for x, y in zip(got, first):
+            np.testing.assert_array_equal(x, y)
+    s.close()
