@@ -1142,7 +1142,8 @@ void pickResident(dg_context* c) {
 }
 
 // A context whose loop handed a batch back launches per stage from then on: what made its blocks wait
-// (another process on the card) tends to last, and every further attempt costs its patience.
+// (another process on the card, or a large context stepping beside it) tends to last, and every further
+// attempt costs its patience.
 bool useResident(const dg_context* c) { return c->resBlocks > 0 && c->resChunk >= kResMinChunk && !c->resOff; }
 
 // Batches of fewer steps are launched per stage: a resident launch costs 50-60 us before its first step
@@ -1158,7 +1159,9 @@ constexpr int kResShortBatches = 16;
 
 // Longest wait of a block for another before a launch is given up, in microseconds. Waits are a few
 // microseconds; a launch whose blocks do not all fit (two processes on one card do not see each other's
-// cooperative launches) would wait for good. Short against what a call takes, long against the
+// cooperative launches) would wait for good, and one beside the back-to-back stage launches of a large
+// grid may as well (18,432 triangles FP64 beside 196,608 tetrahedra on another thread: given up with
+// 20 ms, 100 ms and 2 s alike). Short against what a call takes, long against the
 // dispatch of the last blocks behind other kernels.
 constexpr uint64_t kResPatienceUs = 20000;
 
